@@ -30,7 +30,8 @@ if os.environ.get("IFX_TUNING") == "1":
     LIB = os.path.join(OBJ, "libifx_qgemm.so")
 # Bit-exact kernels: no fp contraction anywhere in these translation units.
 EXACT = {"quantize.hip", "dequant.hip"}
-SOURCES = ["api.hip", "quantize.hip", "dequant.hip", "gemv.hip", "mmq_skinny.hip", "mmvq.hip", "gemm_mfma.hip", "gemv_lds.hip", "gemv_slot.hip", "gemm_f16.hip", "gemv_dq.hip", "packed.hip",
+SOURCES = ["api.hip", "quantize.hip", "dequant.hip", "gemv.hip", "mmq_skinny.hip", "mmvq.hip", "gemm_mfma.hip", "gemv_lds.hip", "gemv_slot.hip", "gemm_f16.hip", "gemm_f16_q4.hip", "gemm_f16_q6.hip", "gemm_f16_q8.hip",
+           "gemv_dq.hip", "packed.hip",
            "../host/fused_quant_gemm.cpp", "../host/native_dispatch.cpp", "../host/gguf.cpp", "../host/gguf_model.cpp"]
 
 
