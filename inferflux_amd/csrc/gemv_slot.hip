@@ -26,9 +26,10 @@
 //         are the two groups: each group gets a slot of its own.
 //
 // Lane mapping.  Lane l supplies weight row c = l % 32 of the wave's 32
-// rows and K half h = l / 32 of every block: a 16-byte chunk of its row's
-// super-block that it loads itself (no LDS for weights; a row's whole
-// super-block is in flight in 64 lanes x 5-7 loads).  For the activation
+// rows and K half h = l / 32 of every block: 16-byte chunks of its row's
+// super-block, loaded in that layout from tiled rows and passed through LDS
+// from raw ones (WRaw); a super-block of 32 rows is in flight in 5-8 loads a
+// lane.  For the activation
 // operand lane l is MFMA row r = l % 32, i.e. batch row r % MP of slot
 // r / MP; it loads the 16 codes of its batch row's block for its slot.
 // The result layout gives lane l weight row c and batch rows
@@ -158,6 +159,57 @@ __device__ __forceinline__ void load_w(WSb<QT> &w, rsrc_t Wr, uint32_t voff, uin
   }
 }
 
+// Raw rows, staged: a lane's row is its own, so loads in the lane layout touch
+// 32 rows each and cost the vector cache an access a lane (a pure read of that
+// pattern reaches 2.2-2.4 TB/s against 5.2 for consecutive lanes on
+// consecutive bytes).  The wave loads its 32 rows' super-blocks along the rows
+// instead, 16-byte piece after piece, and passes them through an area of LDS
+// of its own (in order there: no barrier) into the lane layout.  A row's 9
+// (Q4_K) or 13 pieces are an odd number, so the reads fall on distinct banks.
+// Q6_K's 16 bits of d are loaded by their lanes.  Us raw, before and
+// after: LM head 151936 x 2048 Q6_K at M = 5 / 8 78 / 82 -> 66 / 75, 3B down
+// 2048 x 11008 Q6_K at M = 6 11.0 -> 8.5 (accumulate), 3B gate/up + SiLU at M = 6
+// 11.6 -> 10.8, 3B Q/K/V at M = 6 5.0 -> 4.5 (tiled rows: 54, 6.6-7.4, 9.7, 3.9).
+template <int QT>
+struct WRaw {
+  static constexpr int kPieces = QT == kTypeQ4_K ? 9 : 13;
+  static constexpr int kLoads = (32 * kPieces + 63) / 64;
+  static constexpr int kArea = kLoads * 1024;  // LDS bytes a wave
+  u32x4 p[kLoads];
+  uint32_t d;
+};
+
+template <int QT>
+__device__ __forceinline__ void load_raw(WRaw<QT> &w, rsrc_t Wr, const uint32_t (&voff)[WRaw<QT>::kLoads],
+                                         uint32_t row_off, uint32_t sb_off) {
+#pragma unroll
+  for (int i = 0; i < WRaw<QT>::kLoads; ++i) w.p[i] = wload<u32x4>(Wr, voff[i], sb_off);
+  if constexpr (QT == kTypeQ6_K) w.d = wload<uint16_t>(Wr, row_off + 208, sb_off);
+}
+
+template <int QT>
+__device__ __forceinline__ void raw_to_lanes(WSb<QT> &w, const WRaw<QT> &r, uint8_t *area, int lane) {
+#pragma unroll
+  for (int i = 0; i < WRaw<QT>::kLoads; ++i)
+    *reinterpret_cast<u32x4 *>(area + 1024 * i + 16 * lane) = r.p[i];
+  wave_sync();
+  const uint8_t *row = area + (lane & 31) * 16 * WRaw<QT>::kPieces;
+  const int h = lane >> 5;
+  auto at = [&](int o) { return *reinterpret_cast<const u32x4 *>(row + o); };
+  if constexpr (QT == kTypeQ4_K) {
+    w.hdr = at(0);
+#pragma unroll
+    for (int p = 0; p < 4; ++p) w.q[p] = at(16 + 32 * p + 16 * h);
+  } else {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) w.ql[i] = at(64 * (i >> 1) + 32 * (i & 1) + 16 * h);
+#pragma unroll
+    for (int hf = 0; hf < 2; ++hf) w.qh[hf] = at(128 + 32 * hf + 16 * h);
+    w.sc = at(192);
+    w.d = r.d;
+  }
+}
+
 // a_off[c]: this lane's code offset for chain c within super-block 0 (or an
 // offset past the end of A, which loads zeros); ds_off[u]: table entries.
 template <int QT, int MP>
@@ -198,12 +250,18 @@ __device__ __forceinline__ i32x4 w_operand(const WSb<QT> &w, int j) {
 }  // namespace
 
 // NP: projections per workgroup (2 for the fused gate/up/SiLU launch).
-template <int QT, int MP, int KW, int NP = 1>
+// Whether a launch stages raw rows (16 waves of Q6_K areas would pass 64 KB).
+template <int KW, bool SW, bool TL>
+constexpr bool slot_staged() { return !TL && !(SW && KW == 8); }
+
+template <int QT, int MP, int KW, bool SW, bool TL>
 constexpr int slot_lds_bytes() {
+  constexpr int NP = SW ? 2 : 1;
+  constexpr int raw = slot_staged<KW, SW, TL>() ? NP * KW * WRaw<QT>::kArea : 0;  // first: 16-byte aligned
   constexpr int table = NP * KW * 2 * 8 * MP * 4;                     // per-wave d and s tables
   constexpr int red = NP * (KW > 1 ? KW - 1 : 0) * 64 * (MP / 2) * 4;  // partial results
   constexpr int gu = NP == 2 ? 2 * MP * 32 * 4 : 0;                    // gate/up outputs
-  return table + red + gu;
+  return raw + table + red + gu;
 }
 
 // SW: fused gate/up/SiLU (the reference's FusedGateUpSiluGemvQ8_1,
@@ -227,7 +285,10 @@ __global__ __launch_bounds__(64 * KW * (SW ? 2 : 1)) void k_gemv_slot(const Slot
   using G = SlotGeo<QT, MP>;
   constexpr int NM = G::kNm;
   static_assert(!(SW && SPLIT), "the fused gate/up/SiLU launch does not split K");
-  extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
+  extern __shared__ __attribute__((aligned(16))) uint8_t smem_all[];
+  constexpr bool kStaged = slot_staged<KW, SW, TL>();
+  constexpr int kAreas = kStaged ? (SW ? 2 : 1) * KW * WRaw<QT>::kArea : 0;
+  uint8_t *smem = smem_all + kAreas;  // past the waves' row areas
   const int bx = blockIdx.x;
   const int wave_all = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int proj = SW ? wave_all / KW : 0;  // SW: 0 gate, 1 up
@@ -254,6 +315,13 @@ __global__ __launch_bounds__(64 * KW * (SW ? 2 : 1)) void k_gemv_slot(const Slot
   const uint32_t w_voff = TL ? 16u * c32 : static_cast<uint32_t>(min(n0 + c32, N - 1)) * w_row;
   const uint32_t w_soff = TL ? static_cast<uint32_t>(n0 / 32) * nsb * kTile : 0u;  // group's first tile
   constexpr int kSbStep = TL ? kTile : kSbBytes;  // bytes between a row's super-blocks
+  uint8_t *area = smem_all + wave_all * (kStaged ? WRaw<QT>::kArea : 0);
+  uint32_t r_off[WRaw<QT>::kLoads];  // staged: this lane's piece of load i (past row 31: row 31's)
+#pragma unroll
+  for (int i = 0; i < WRaw<QT>::kLoads; ++i) {
+    const int e = 64 * i + lane, r = min(e / WRaw<QT>::kPieces, 31);
+    r_off[i] = static_cast<uint32_t>(min(n0 + r, N - 1)) * w_row + 16 * (e % WRaw<QT>::kPieces);
+  }
   // activation operand: MFMA row r = c32 = batch row (r % MP) of slot r / MP
   const int am = c32 % MP, aslot = c32 / MP;
   bool a_valid = true;
@@ -304,19 +372,24 @@ __global__ __launch_bounds__(64 * KW * (SW ? 2 : 1)) void k_gemv_slot(const Slot
   const int step = kSplitK ? KW * static_cast<int>(gridDim.y) : KW;
   int sb = (kSplitK ? static_cast<int>(blockIdx.y) * KW : 0) + wave;
   WSb<QT> wc;
+  WRaw<QT> rc;
   ASb<QT, MP> ac;
   if (sb < nsb) {
-    load_w<QT, TL>(wc, Wr, w_voff, w_soff + sb * kSbStep, h);
+    if constexpr (kStaged) load_raw<QT>(rc, Wr, r_off, w_voff, sb * kSbStep);
+    else load_w<QT, TL>(wc, Wr, w_voff, w_soff + sb * kSbStep, h);
     load_a<QT, MP>(ac, Ar, a_off, ds_off, sb * 8 * kQ8_1Bytes);
   }
   for (; sb < nsb; sb += step) {
     WSb<QT> wn;
+    WRaw<QT> rn;
     ASb<QT, MP> an;
     const bool more = sb + step < nsb;
     if (more) {
-      load_w<QT, TL>(wn, Wr, w_voff, w_soff + (sb + step) * kSbStep, h);
+      if constexpr (kStaged) load_raw<QT>(rn, Wr, r_off, w_voff, (sb + step) * kSbStep);
+      else load_w<QT, TL>(wn, Wr, w_voff, w_soff + (sb + step) * kSbStep, h);
       load_a<QT, MP>(an, Ar, a_off, ds_off, (sb + step) * 8 * kQ8_1Bytes);
     }
+    if constexpr (kStaged) raw_to_lanes<QT>(wc, rc, area, lane);
     // d and s of this super-block's 8 x MP activation blocks
 #pragma unroll
     for (int u = 0; u < MP / 8; ++u) {
@@ -423,7 +496,8 @@ __global__ __launch_bounds__(64 * KW * (SW ? 2 : 1)) void k_gemv_slot(const Slot
     }
     wave_sync();  // table reads precede the next super-block's writes
     if (more) {
-      wc = wn;
+      if constexpr (kStaged) rc = rn;
+      else wc = wn;
       ac = an;
     }
   }
@@ -598,7 +672,7 @@ void choose_slot_work(int blocks, int nsb, bool no_split, int &kw, int &ks) {
 
 template <int QT, int MP, int KW, bool F16OUT, int SPLIT, bool TL>
 void slot_launch(const SlotArgs &args, int blocks, int ks, hipStream_t s) {
-  constexpr int lds = slot_lds_bytes<QT, MP, KW>();
+  constexpr int lds = slot_lds_bytes<QT, MP, KW, false, TL>();
   if constexpr (TL)
     IFX_LAUNCH(k_gemv_slot, (QT, MP, KW, F16OUT, SPLIT, false, true), dim3(blocks, ks),
                dim3(64 * KW), lds, s, args);
@@ -664,7 +738,7 @@ void slot_q(const SlotArgs &args, int blocks, bool f16, hipStream_t s) {
 // IFX_SLOT_KW overrides, as for the plain launch.
 template <int QT, int MP, int KW, bool TL>
 void slot_swiglu_launch(const SlotArgs &args, bool f16h, hipStream_t s) {
-  constexpr int lds = slot_lds_bytes<QT, MP, KW, 2>();
+  constexpr int lds = slot_lds_bytes<QT, MP, KW, true, TL>();
   const dim3 grid(args.seg[0].N / 32);
   if constexpr (TL) {
     if (f16h) IFX_LAUNCH(k_gemv_slot, (QT, MP, KW, true, false, true, true), grid, dim3(128 * KW), lds, s, args);
