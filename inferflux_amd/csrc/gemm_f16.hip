@@ -93,9 +93,27 @@ struct Plan {
   int tile, m_tiles, n_tiles, splits, spw;
 };
 
+// Most K splits that a shape may take: as many as fill the chip once over a
+// grid of 256 x 256 tiles, keeping 512 values of K each.  This line is part
+// of the interface and does not move with the tiles: it says which shapes
+// need the ordered reduction's workspace and how much, and which give the
+// same bits on every run without it.
+int max_splits(int count, const int *N, int M, int K) {
+  const int nch = K / 64;
+  int most = 256;
+  for (int i = 0; i < count; ++i) {
+    const int64_t tiles = int64_t{1} * ((M + 255) / 256) * ((N[i] + 255) / 256);
+    int sp = tiles < 192 ? std::max(1, std::min(static_cast<int>(256 / tiles), nch / 8)) : 1;
+    const int each = (nch + sp - 1) / sp;
+    sp = (nch + each - 1) / each;
+    most = std::min(most, sp);
+  }
+  return most;
+}
+
 // Tile and K splits of a launch: the cheapest by the table.  Only fp32 outputs
 // split (their partial sums meet in Y by atomics, or in slots), when the tiles
-// alone do not fill the CUs, down to 512 values a split; the reduction adds
+// alone do not fill the CUs, up to max_splits; the reduction adds
 // about 4 us and 0.5 us a megabyte of partial sums.  A launch that would leave
 // three quarters of the CUs idle always splits.  splits_req > 0 forces the
 // count (tests; at most one split per group of stages).
@@ -106,6 +124,7 @@ Plan f16_plan(int qt, bool f16, int count, const int *N, int M, int K, int split
     const char *e = tuning_env("IFX_F16_TILE");
     return e ? atoi(e) : -1;
   }();
+  const int cap = f16 ? 1 : max_splits(count, N, M, K);
   int64_t n_sum = 0;
   for (int i = 0; i < count; ++i) n_sum += N[i];
   Plan best{};
@@ -123,7 +142,7 @@ Plan f16_plan(int qt, bool f16, int count, const int *N, int M, int K, int split
     const int kc = t.kw * (qt == kTypeQ8_0 ? 1 : 2);  // chunks of a group
     const int groups = (nch + kc - 1) / kc;
     int most = 1;
-    if (!f16 && wg < 192) most = static_cast<int>(std::max<int64_t>(1, std::min<int64_t>(256 / wg, nch / 8)));
+    if (!f16 && wg < 192) most = std::max(1, std::min(static_cast<int>(256 / wg), cap));
     int least = most > 1 && wg <= 64 ? 2 : 1;
     if (splits_req > 0 && !f16) least = most = splits_req;
     for (int sp = least; sp <= most; ++sp) {
