@@ -156,8 +156,8 @@ int ifx_qgemv(int quant_type, const void *W, const void *A_q8_1, void *Y, int ou
 /* count (1..3) sibling projections of one quant type that read the same
  * Q8_1 activations, e.g. gate + up or Q + K + V: y_i (op)= W_i . a with
  * W_i [N[i]][K] and Y_i [M][N[i]].  For M <= 2 this is one launch whose
- * workgroups walk the rows of all projections; larger M runs one MFMA
- * launch per projection.  mode: IFX_STORE or IFX_ACCUM (no bias).  W, Y and
+ * workgroups walk the rows of all projections, and so do the MFMA launches of
+ * larger M.  mode: IFX_STORE or IFX_ACCUM (no bias).  W, Y and
  * N are host arrays of count entries.
  * Replaces FusedQuantGemm::GemvQ8_1Pair / GemvQ8_1Triple
  * (fused_quant_gemm.h:272-276, 309-313; kernels mmvq.cuh:1197-1448). */
@@ -262,7 +262,7 @@ int ifx_qgemm_prefill(int quant_type, const void *W, const void *A_q8_1, void *Y
 /* Bytes of caller-owned workspace ifx_qgemm_prefill_ws uses at this shape
  * (the fp16 copy of the activations, M x K halves), or 0 when the prefill
  * GEMM at this shape does not use one: below the fp16 GEMM's range, or
- * N < 16384, where too few weight tiles share the copy for it to pay. */
+ * N < 16384, where too few weight tiles share the copy. */
 int64_t ifx_qgemm_prefill_workspace_bytes(int quant_type, int M, int N, int K);
 
 /* ifx_qgemm_prefill with a caller-owned workspace (16-byte aligned, at least
@@ -280,7 +280,7 @@ int ifx_qgemm_prefill_ws(int quant_type, const void *W, const void *A_q8_1, void
 
 /* Deterministic prefill: ifx_qgemm_prefill_ws whose K split (fp32 outputs
  * of shapes with too few output tiles to fill the GPU, e.g. Q6_K
- * 5120 x 27648 at M = 512: six splits) stores each split's fp32 tile in its
+ * 5120 x 27648 at M = 512) stores each split's fp32 tile in its
  * own workspace slot and adds the slots in split order in a second launch,
  * with no zero fill and no fp32 atomics: the same bits on every call.
  * Workspace: at least ifx_qgemm_prefill_ordered_workspace_bytes bytes,

@@ -43,6 +43,9 @@ hipError_t launch_mmq_skinny(int qtype, int count, const void *const *W, void *c
                              int K, int mode, hipStream_t stream);
 hipError_t launch_gemm_mfma(int qtype, const void *W, const void *A, void *Y, const void *bias,
                             bool f16, int M, int N, int K, int mode, hipStream_t stream);
+hipError_t launch_gemm_mfma_grouped(int qtype, int count, const void *const *W, const void *A,
+                                    void *const *Y, const int *N, const void *bias, bool f16,
+                                    int M, int K, int mode, hipStream_t stream);
 bool gemv_lds_fits(int qtype, int M, int K);
 hipError_t launch_gemv_lds(int count, const void *const *W, void *const *Y, const int *N,
                            const void *bias, const void *A, bool f16, int M, int K, int mode,
@@ -141,8 +144,9 @@ constexpr int kMaxSkinnyM = 32;
 // us for fp16 / int8): Q6_K 5120 x 27648 M = 48: 111 / 438, M = 128: 118 /
 // 438 (the int8 kernel's per-block rescale of 16-value Q6_K groups); Q4_K
 // 27648 x 5120 M = 48: 104 / 63, M = 64: 98 / 64, M = 96: 99 / 105, M = 128:
-// 102 / 104.  Q8_0 is unmeasured and keeps 128 (a 256-row tile is mostly
-// padding below that).  IFX_PREFILL=int8|f16 forces one (tuning; read once).
+// 102 / 104 (fp16 on a 256 x 256 tile).  Batches under the lines keep the
+// integer-exact sums whatever the fp16 kernel's time.  IFX_PREFILL=int8|f16
+// forces one (tuning; read once).
 int min_f16_gemm_m(int qtype) {
   return qtype == IFX_TYPE_Q6_K ? kMaxSkinnyM + 1 : qtype == IFX_TYPE_Q4_K ? 96 : 128;
 }
@@ -303,7 +307,7 @@ int check_gemm_args(int quant_type, const void *W, const void *A, void *Y, int o
 // or the split's ordered reduction, costs more than it gains), and so do
 // narrow launches (integer-exact sums: a row of few outputs is no norm to
 // hide the fp16 weight rounding behind).
-enum class Route { F16Gemm, Gemv, Lds, Slot, Dq, Skinny, Mmvq, Mfma, PerProjection };
+enum class Route { F16Gemm, Gemv, Lds, Slot, Dq, Skinny, Mmvq, Mfma };
 Route route(int qt, int M, int K, int n_total, bool f16, bool grouped, bool atomic_accum = false) {
   static const int acc_min_m = [] {  // IFX_ACCUM_DQ_MIN_M (tuning; read once)
     const char *e = ifx::tuning_env("IFX_ACCUM_DQ_MIN_M");
@@ -327,14 +331,15 @@ Route route(int qt, int M, int K, int n_total, bool f16, bool grouped, bool atom
       return Route::Slot;
     return Route::Dq;
   }
-  if (!grouped && !gemv_only(qt) && M > kMaxSkinnyM && use_f16_gemm(qt, M, K)) return Route::F16Gemm;
+  if (!gemv_only(qt) && M > kMaxSkinnyM && (!grouped || K % 256 == 0) && use_f16_gemm(qt, M, K))
+    return Route::F16Gemm;
   if (gemv_only(qt) || row_split(qt) || M <= max_gemv_m() || (M > kMaxSkinnyM && K % 256 != 0))
     return Route::Gemv;
   if (use_lds(qt, M, K, n_total)) return Route::Lds;
   if (use_slot(qt, M, K, n_total, f16)) return Route::Slot;
   if (use_dq(qt, M, K, f16)) return Route::Dq;
   if (M <= kMaxSkinnyM) return (use_skinny(M) && K % 256 == 0) ? Route::Skinny : Route::Mmvq;
-  return grouped ? Route::PerProjection : Route::Mfma;
+  return Route::Mfma;
 }
 
 // The ordered-split workspace of a slot / dq launch: nullptr when there is
@@ -433,22 +438,16 @@ int grouped_impl(int quant_type, int count, const void *const *W, void *const *Y
   case Route::Mmvq:
     return status_of(ifx::launch_mmvq(quant_type, count, W, Y, N, nullptr, A_q8_1, f16, M, K,
                                       mode, s));
-  default:
-    break;
-  }
-  // prefill: the projections' tiles share a launch, so that narrow ones (K and
-  // V) do not each leave most of the CUs idle (14B K or V at M = 512: 17 us
-  // alone of the 58 us that Q/K/V take together)
-  if (use_f16_gemm(quant_type, M, K) && M > kMaxSkinnyM)
+  // prefill and larger batches: the projections' tiles share a launch, so that
+  // narrow ones (K and V) do not each leave most of the CUs idle (14B K or V
+  // at M = 512: 17 us alone of the 58 us that Q/K/V take together)
+  case Route::F16Gemm:
     return status_of(ifx::launch_gemm_f16_grouped(quant_type, count, W, A_q8_1, nullptr, Y, N,
                                                   nullptr, f16, M, K, mode, 0, s));
-  // larger decode batches: one launch per projection
-  for (int i = 0; i < count; ++i) {
-    const int rc = qgemv_impl(quant_type, W[i], A_q8_1, Y[i], out_dtype, mode, nullptr, M, N[i],
-                              K, stream, ws, ws_bytes, ordered);
-    if (rc != IFX_OK) return rc;
+  default:
+    return status_of(ifx::launch_gemm_mfma_grouped(quant_type, count, W, A_q8_1, Y, N, nullptr,
+                                                   f16, M, K, mode, s));
   }
-  return IFX_OK;
 }
 
 }  // namespace
@@ -789,9 +788,10 @@ int ifx_qgemm_prefill(int quant_type, const void *W, const void *A_q8_1, void *Y
   return status_of(ifx::launch_gemm_mfma(quant_type, W, A_q8_1, Y, bias, f16, M, N, K, mode, s));
 }
 
-// The fp16 copy pays where many weight tiles share it: measured at M = 512,
-// Q4_K 27648 x 5120 (108 tiles of 256 columns) 190 -> 162 us, Q6_K
-// 5120 x 27648 (20 tiles) 234 -> 250 us.
+// The fp16 copy is used where many weight tiles share it.  The line is part
+// of the interface (callers size their workspace by it); on the present tiles
+// the GEMM takes the same time with it and without (Q4_K 27648 x 5120 at
+// M = 512: 163 us), on few tiles the copy's own launch costs more.
 constexpr int kMinWorkspaceN = 16384;
 
 int64_t ifx_qgemm_prefill_workspace_bytes(int quant_type, int M, int N, int K) {

@@ -11,10 +11,10 @@
 // group for Q6_K), then fp32 scaling by the weight and activation block
 // scales -- with the integer dot on the matrix cores.
 //
-// Tiling: a 256-thread workgroup owns a 128 (m) x 128 (n) output tile (64 x
-// 64 when that gives fewer than two workgroups per CU); its four waves are
-// 2 x 2, each owning 2 x 2 (or one) MFMA tiles of 32 x 32.
-// The K loop steps one 256-value super-block at a time:
+// Tiling: a workgroup of one to four 256-thread groups owns a 128 (m) x 128 (n) output tile (64 x
+// 64 when that gives fewer than two workgroups per CU); a group's four waves
+// are 2 x 2, each owning 2 x 2 (or one) MFMA tiles of 32 x 32.
+// A group's K loop steps one 256-value super-block at a time:
 //   1. the next super-block's A items (Q8_1 blocks of 128 rows) and raw W
 //      bytes (16-byte chunks of 128 rows) are loaded into registers while
 //      the current one is computed; at the top of a step they are written
@@ -152,7 +152,8 @@ __device__ __forceinline__ void fetch(Prefetch<QT, S> &pf, rsrc_t Wr, rsrc_t Ar,
 }
 
 template <int QT, int S>
-__device__ __forceinline__ void commit(Smem<QT, S> &sm, const Prefetch<QT, S> &pf, int tid) {
+__device__ __forceinline__ void commit(Smem<QT, S> &sm, const Prefetch<QT, S> &pf,
+                                       int tid) {
   constexpr int kBN = Prefetch<QT, S>::kBN;
 #pragma unroll
   for (int i = 0; i < Prefetch<QT, S>::kAItems; ++i) {
@@ -185,23 +186,51 @@ __device__ __forceinline__ void commit(Smem<QT, S> &sm, const Prefetch<QT, S> &p
   }
 }
 
+constexpr int kMaxSeg = 3;
+
+// A projection of the launch: its weights, output, rows, and the n tile that
+// ends it.
+struct MfmaSeg {
+  const uint8_t *W;
+  void *Y;
+  int N, end;
+};
+struct MfmaArgs {
+  MfmaSeg seg[kMaxSeg];
+  const uint8_t *A;
+  const void *bias;
+  int M, K, mode;
+};
+
 }  // namespace
 
-template <int QT, int S, bool F16OUT>
-__global__ __launch_bounds__(256, 2) void k_gemm_mfma(const uint8_t *__restrict__ W,
-                                                      const uint8_t *__restrict__ A,
-                                                      void *__restrict__ Y,
-                                                      const void *__restrict__ bias, int M,
-                                                      int N, int K, int mode) {
+// KW groups of four waves share an output tile: group g walks super-blocks
+// g, g + KW, ... with an LDS stage of its own, and the groups' sums meet in
+// LDS in group order (no atomics; the same bits on every run).  Bound by the
+// VALU (three operations per output and block: 9 us of a CU for one 64 x 64
+// tile over K = 2048) and, with one group, by each step's load that a single
+// wave per SIMD cannot hide.  A launch takes up to three projections of the
+// same activations: 3B gate and up (11008 x 2048 Q4_K) at M = 60, two
+// launches 42 us, one 26.
+template <int QT, int S, bool F16OUT, int KW>
+__global__ __launch_bounds__(256 * KW, KW == 1 ? 2 : 4) void k_gemm_mfma(MfmaArgs g) {
   using F = GFmt<QT>;
   extern __shared__ __attribute__((aligned(16))) uint8_t smem_raw[];
-  Smem<QT, S> &sm = *reinterpret_cast<Smem<QT, S> *>(smem_raw);
   constexpr int kBM = 64 * S, kBN = 64 * S;
-  const int tid = threadIdx.x;
+  const int kg = KW == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x >> 8);
+  Smem<QT, S> &sm = reinterpret_cast<Smem<QT, S> *>(smem_raw)[kg];
+  const int tid = threadIdx.x & 255;
   const int lane = tid & 63;
   const int wave = tid >> 6;
+  const int bx = blockIdx.x;
+  const int sg = (bx >= g.seg[0].end) + (bx >= g.seg[1].end);
+  const uint8_t *W = g.seg[sg].W, *A = g.A;
+  void *Y = g.seg[sg].Y;
+  const void *bias = g.bias;
+  const int M = g.M, N = g.seg[sg].N, K = g.K, mode = g.mode;
+  const int nt = bx - (sg ? g.seg[sg - 1].end : 0);
   const int wm = wave & 1, wn = wave >> 1;  // wave position in the 2 x 2 grid
-  const int m0 = blockIdx.y * kBM, n0 = blockIdx.x * kBN;
+  const int m0 = blockIdx.y * kBM, n0 = nt * kBN;
   const int l32 = lane & 31, h = lane >> 5;
   const int nblk32 = K >> 5;
   const uint32_t a_row = static_cast<uint32_t>(nblk32) * kQ8_1Bytes;
@@ -230,12 +259,17 @@ __global__ __launch_bounds__(256, 2) void k_gemm_mfma(const uint8_t *__restrict_
 
   const int nsteps = K >> 8;
   Prefetch<QT, S> pf;
-  fetch<QT, S>(pf, Wr, Ar, w_row, a_row, m0, n0, M, N, 0, tid);
-  for (int sblk = 0; sblk < nsteps; ++sblk) {
+  // a group past the last super-block loads the last one again and adds
+  // nothing (every wave meets every barrier)
+  fetch<QT, S>(pf, Wr, Ar, w_row, a_row, m0, n0, M, N, min(kg, nsteps - 1), tid);
+  for (int s0 = 0; s0 < nsteps; s0 += KW) {
+    const int sblk = s0 + kg;
     __syncthreads();  // previous step's LDS reads are done
     commit<QT, S>(sm, pf, tid);
     __syncthreads();
-    if (sblk + 1 < nsteps) fetch<QT, S>(pf, Wr, Ar, w_row, a_row, m0, n0, M, N, sblk + 1, tid);
+    if (s0 + KW < nsteps)
+      fetch<QT, S>(pf, Wr, Ar, w_row, a_row, m0, n0, M, N, min(sblk + KW, nsteps - 1), tid);
+    if (KW > 1 && sblk >= nsteps) continue;
 
     if constexpr (QT == kTypeQ4_K) {
       float dsc[S][8];
@@ -321,7 +355,7 @@ __global__ __launch_bounds__(256, 2) void k_gemm_mfma(const uint8_t *__restrict_
           // 16-value group u (0/1): values 16u..16u+15 of this 32-run; this
           // lane supplies values 16u + 8h .. 16u + 8h + 7.
           int64_t bq[S][2];
-          int s0[S], s1[S];
+          int sc0[S], sc1[S];
 #pragma unroll
           for (int t = 0; t < S; ++t) {
             const uint8_t *row = &sm.w[bn[t] * F::kPitch];
@@ -338,8 +372,8 @@ __global__ __launch_bounds__(256, 2) void k_gemm_mfma(const uint8_t *__restrict_
             }
             // scales[g*8 + 2*sub + u]
             const uint32_t sw = scw[t][2 * g + (sub >> 1)] >> (16 * (sub & 1));
-            s0[t] = static_cast<int8_t>(sw & 0xFFu);
-            s1[t] = static_cast<int8_t>((sw >> 8) & 0xFFu);
+            sc0[t] = static_cast<int8_t>(sw & 0xFFu);
+            sc1[t] = static_cast<int8_t>((sw >> 8) & 0xFFu);
           }
 #pragma unroll
           for (int s = 0; s < S; ++s) {
@@ -358,7 +392,7 @@ __global__ __launch_bounds__(256, 2) void k_gemm_mfma(const uint8_t *__restrict_
               const float dd = dq[t];
 #pragma unroll
               for (int i = 0; i < 16; ++i) {
-                const int ci = __mul24(c0[i], s0[t]) + __mul24(c1[i], s1[t]);
+                const int ci = __mul24(c0[i], sc0[t]) + __mul24(c1[i], sc1[t]);
                 acc[s][t][i] += static_cast<float>(ci) * (fa[i >> 2][i & 3] * dd);
               }
             }
@@ -394,6 +428,36 @@ __global__ __launch_bounds__(256, 2) void k_gemm_mfma(const uint8_t *__restrict_
     }
   }
 
+  // The groups' sums meet in LDS; group g then owns 16 / KW of each tile's
+  // values.
+  constexpr int kOwn = 16 / KW;
+  if constexpr (KW > 1) {
+    float *part = reinterpret_cast<float *>(smem_raw);  // [group][t, s, i][thread]
+    constexpr int kVals = S * S * 16;
+    static_assert(kVals * 256 * 4 <= sizeof(Smem<QT, S>), "the sums reuse the stages");
+    __syncthreads();
+#pragma unroll
+    for (int s = 0; s < S; ++s)
+#pragma unroll
+      for (int t = 0; t < S; ++t)
+#pragma unroll
+        for (int i = 0; i < 16; ++i)
+          part[(kg * kVals + (s * S + t) * 16 + i) * 256 + tid] = acc[s][t][i];
+    __syncthreads();
+#pragma unroll
+    for (int s = 0; s < S; ++s)
+#pragma unroll
+      for (int t = 0; t < S; ++t)
+#pragma unroll
+        for (int i = 0; i < kOwn; ++i) {
+          const int v = (s * S + t) * 16 + kg * kOwn + i;
+          float sum = part[v * 256 + tid];
+#pragma unroll
+          for (int k = 1; k < KW; ++k) sum += part[(k * kVals + v) * 256 + tid];
+          acc[s][t][i] = sum;
+        }
+  }
+
   // Epilogue: lane holds column n and rows rbase + 8g + j.
 #pragma unroll
   for (int s = 0; s < S; ++s)
@@ -402,8 +466,9 @@ __global__ __launch_bounds__(256, 2) void k_gemm_mfma(const uint8_t *__restrict_
       const int n = n0 + wn * 32 * S + 32 * t + l32;
       if (n >= N) continue;
 #pragma unroll
-      for (int i = 0; i < 16; ++i) {
-        const int m = m0 + wm * 32 * S + 32 * s + 8 * (i >> 2) + 4 * h + (i & 3);
+      for (int i = 0; i < kOwn; ++i) {
+        const int v = kg * kOwn + i;
+        const int m = m0 + wm * 32 * S + 32 * s + 8 * (v >> 2) + 4 * h + (v & 3);
         if (m >= M) continue;
         const int64_t o = static_cast<int64_t>(m) * N + n;
         float y = acc[s][t][i];
@@ -422,39 +487,62 @@ __global__ __launch_bounds__(256, 2) void k_gemm_mfma(const uint8_t *__restrict_
     }
 }
 
-template <int QT, int S>
-static hipError_t launch_qts(const uint8_t *W, const uint8_t *A, void *Y, const void *bias,
-                             bool f16, int M, int N, int K, int mode, hipStream_t s) {
-  constexpr int kB = 64 * S;
-  const dim3 grid((N + kB - 1) / kB, (M + kB - 1) / kB);
-  const size_t shm = sizeof(Smem<QT, S>);
+template <int QT, int S, bool F16OUT, int KW>
+static hipError_t launch_k(const MfmaArgs &g, dim3 grid, hipStream_t s) {
+  const size_t shm = KW * sizeof(Smem<QT, S>);
+  // The log names the type, the tile and the output, not KW.
+  if (!note_launch("k_gemm_mfma", {QT, S, F16OUT})) return hipSuccess;
   // The staged tiles can exceed the 64 KiB default; gfx950 has 160 KiB of LDS.
-  // set once per kernel (function-local statics: thread-safe)
-  if (!dry_run()) {
-    static const hipError_t attr_f32 = hipFuncSetAttribute(
-        reinterpret_cast<const void *>(&k_gemm_mfma<QT, S, false>),
-        hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(shm));
-    static const hipError_t attr_f16 = hipFuncSetAttribute(
-        reinterpret_cast<const void *>(&k_gemm_mfma<QT, S, true>),
-        hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(shm));
-    const hipError_t attr = f16 ? attr_f16 : attr_f32;
-    if (attr != hipSuccess) return attr;
-  }
-  if (f16)
-    IFX_LAUNCH(k_gemm_mfma, (QT, S, true), grid, dim3(256), shm, s, W, A, Y, bias, M, N, K, mode);
-  else
-    IFX_LAUNCH(k_gemm_mfma, (QT, S, false), grid, dim3(256), shm, s, W, A, Y, bias, M, N, K, mode);
+  // set once per kernel (function-local static: thread-safe)
+  static const hipError_t attr = hipFuncSetAttribute(
+      reinterpret_cast<const void *>(&k_gemm_mfma<QT, S, F16OUT, KW>),
+      hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(shm));
+  if (attr != hipSuccess) return attr;
+  hipLaunchKernelGGL((k_gemm_mfma<QT, S, F16OUT, KW>), grid, dim3(256 * KW), shm, s, g);
   return last_error();
 }
 
-// 128 x 128 workgroup tiles when they give at least two workgroups per CU,
-// else 64 x 64 (e.g. N = 5120 at M = 512: 160 large tiles, 640 small).
+template <int QT, int S, int KW>
+static hipError_t launch_s(MfmaArgs &g, int count, bool f16, hipStream_t s) {
+  constexpr int kB = 64 * S;
+  int end = 0;
+  for (int i = 0; i < kMaxSeg; ++i) {
+    if (i < count) end += (g.seg[i].N + kB - 1) / kB;
+    g.seg[i].end = end;
+  }
+  const dim3 grid(end, (g.M + kB - 1) / kB);
+  return f16 ? launch_k<QT, S, true, KW>(g, grid, s) : launch_k<QT, S, false, KW>(g, grid, s);
+}
+
+// 128 x 128 workgroup tiles when they give at least two workgroups per CU
+// and the batch fills more than half of their rows (LM head 151936 x 2048 at
+// M = 60, large / small tiles: Q4_K 167 / 99 us, Q8_0 177 / 115), else 64 x 64
+// (e.g. N = 5120 at M = 512: 160 large tiles, 640 small).  With no more small
+// tiles than CUs, four groups of waves share each; up to two tiles a CU, two
+// groups.  us for 1 / 2 / 4 groups:
+//   Q4_K 11008 x 2048 at M = 60 (172 tiles)      20.9 / 17.0 / 16.1
+//   Q4_K 13824 x 5120 at M = 64 (216)            45.3 / 35.5 / 32.6
+//   Q4_K 22016 x 2048 at M = 60 (344)            27.3 / 26.3 / 30.4
+//   Q4_K 27648 x 5120 at M = 64 (432)            60.3 / 54.1 / 60.2
+//   Q8_0 2048 x 11008 at M = 60 (32)             93.5 / 81.4 / 74.9
+//   Q8_0 22016 x 2048 at M = 64 (344)            27.6 / 29.6 / 33.7
+//   Q8_0 13824 x 5120 at M = 127 (432)           61.2 / 57.3 / 65.9
+// so Q8_0 (less unpacking to hide the loads behind) takes two groups only
+// from K = 4096 on.  Q6_K runs here on request only and keeps one group.
 template <int QT>
-static hipError_t launch_qt(const uint8_t *W, const uint8_t *A, void *Y, const void *bias, bool f16,
-                            int M, int N, int K, int mode, hipStream_t s) {
-  const int64_t big = static_cast<int64_t>((N + 127) / 128) * ((M + 127) / 128);
-  if (big >= 512) return launch_qts<QT, 2>(W, A, Y, bias, f16, M, N, K, mode, s);
-  return launch_qts<QT, 1>(W, A, Y, bias, f16, M, N, K, mode, s);
+static hipError_t launch_qt(MfmaArgs &g, int count, bool f16, hipStream_t s) {
+  int64_t big = 0, small = 0;
+  for (int i = 0; i < count; ++i) {
+    big += static_cast<int64_t>((g.seg[i].N + 127) / 128) * ((g.M + 127) / 128);
+    small += static_cast<int64_t>((g.seg[i].N + 63) / 64) * ((g.M + 63) / 64);
+  }
+  if (big >= 512 && g.M > 64) return launch_s<QT, 2, 1>(g, count, f16, s);
+  if constexpr (QT != kTypeQ6_K) {
+    if (small <= 256) return launch_s<QT, 1, 4>(g, count, f16, s);
+    if (small <= 512 && (QT == kTypeQ4_K || g.K >= 4096))
+      return launch_s<QT, 1, 2>(g, count, f16, s);
+  }
+  return launch_s<QT, 1, 1>(g, count, f16, s);
 }
 
 hipError_t launch_gemv(int qtype, const void *W, const void *A, void *Y, const void *bias,
@@ -462,17 +550,37 @@ hipError_t launch_gemv(int qtype, const void *W, const void *A, void *Y, const v
 
 // K % 256 == 0 is required for the super-block K loop; Q8_0 weights with
 // K % 256 != 0 run on the GEMV kernel in groups of 8 columns instead.
-hipError_t launch_gemm_mfma(int qtype, const void *W, const void *A, void *Y, const void *bias,
-                            bool f16, int M, int N, int K, int mode, hipStream_t stream) {
-  const uint8_t *w = static_cast<const uint8_t *>(W);
-  const uint8_t *a = static_cast<const uint8_t *>(A);
-  if (K % 256 != 0) return launch_gemv(qtype, W, A, Y, bias, f16, M, N, K, mode, stream);
+hipError_t launch_gemm_mfma_grouped(int qtype, int count, const void *const *W, const void *A,
+                                    void *const *Y, const int *N, const void *bias, bool f16,
+                                    int M, int K, int mode, hipStream_t stream) {
+  if (K % 256 != 0) {
+    for (int i = 0; i < count; ++i) {
+      const hipError_t e = launch_gemv(qtype, W[i], A, Y[i], bias, f16, M, N[i], K, mode, stream);
+      if (e != hipSuccess) return e;
+    }
+    return hipSuccess;
+  }
+  MfmaArgs g{};
+  for (int i = 0; i < kMaxSeg; ++i) {
+    const int k = i < count ? i : count - 1;
+    g.seg[i] = {static_cast<const uint8_t *>(W[k]), Y[k], N[k], 0};
+  }
+  g.A = static_cast<const uint8_t *>(A);
+  g.bias = bias;
+  g.M = M;
+  g.K = K;
+  g.mode = mode;
   switch (qtype) {
-  case kTypeQ4_K: return launch_qt<kTypeQ4_K>(w, a, Y, bias, f16, M, N, K, mode, stream);
-  case kTypeQ6_K: return launch_qt<kTypeQ6_K>(w, a, Y, bias, f16, M, N, K, mode, stream);
-  case kTypeQ8_0: return launch_qt<kTypeQ8_0>(w, a, Y, bias, f16, M, N, K, mode, stream);
+  case kTypeQ4_K: return launch_qt<kTypeQ4_K>(g, count, f16, stream);
+  case kTypeQ6_K: return launch_qt<kTypeQ6_K>(g, count, f16, stream);
+  case kTypeQ8_0: return launch_qt<kTypeQ8_0>(g, count, f16, stream);
   default: return hipErrorInvalidValue;
   }
+}
+
+hipError_t launch_gemm_mfma(int qtype, const void *W, const void *A, void *Y, const void *bias,
+                            bool f16, int M, int N, int K, int mode, hipStream_t stream) {
+  return launch_gemm_mfma_grouped(qtype, 1, &W, A, &Y, &N, bias, f16, M, K, mode, stream);
 }
 
 }  // namespace ifx
