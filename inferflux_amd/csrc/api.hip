@@ -790,8 +790,8 @@ int ifx_qgemm_prefill(int quant_type, const void *W, const void *A_q8_1, void *Y
 
 // The fp16 copy is used where many weight tiles share it.  The line is part
 // of the interface (callers size their workspace by it); on the present tiles
-// the GEMM takes the same time with it and without (Q4_K 27648 x 5120 at
-// M = 512: 163 us), on few tiles the copy's own launch costs more.
+// the GEMM gains little by it (Q4_K 27648 x 5120 at M = 512: 163-171 us
+// without, 162 with), on few tiles the copy's own launch costs more.
 constexpr int kMinWorkspaceN = 16384;
 
 int64_t ifx_qgemm_prefill_workspace_bytes(int quant_type, int M, int N, int K) {

@@ -312,8 +312,8 @@ def qgemm_prefill_kernel(qtype, W, A, M, N, K, kernel, splits=0, out=None,
 
 def qgemv_grouped(qtype, Ws, A, M, Ns, K, outs=None, out_dtype=torch.float32, mode=STORE,
                   stream=None, workspace=None):
-    """Sibling projections over one Q8_1 A: [W_i . a for W_i in Ws], one launch
-    for M <= 2.  Returns the list of outputs [M, N_i]."""
+    """Sibling projections over one Q8_1 A: [W_i . a for W_i in Ws], one launch.
+    Returns the list of outputs [M, N_i]."""
     import ctypes
     count = len(Ws)
     if not 1 <= count <= 3 or len(Ns) != count:
