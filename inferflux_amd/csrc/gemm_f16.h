@@ -202,14 +202,17 @@ __device__ __forceinline__ void commit_a(_Float16 *chunk, const RawA<AH> &r, int
 // rows that way costs the vector cache an access a lane and the L2 a request
 // for every 32 bytes of a line.  Each wave stages the rows of its own MFMA
 // tiles, one or two chunks (a unit) at a time; no other wave reads them, so no barrier
-// guards them.  A staged row holds its codes in 16-byte pieces, then its fp16
-// scales:
-//   Q4_K  piece 2 ch + h: qs bytes 16 h .. +15 of chunk ch (both nibbles);
-//         8 bytes a chunk: (d sc0, d sc1), (dmin m0, dmin m1)
+// guards them.  A staged row holds its codes in 16-byte pieces, one or two for
+// each K half h, then its fp16 scales.  A piece is 8 bytes from 8 h on and 8
+// from 16 + 8 h on, so that slot sl of a chunk multiplies its values 16 sl ..
+// + 15: the sum of an output runs over K in order, 16 values at a time, on
+// every tile whose waves do not split K.
+//   Q4_K  piece 2 ch + h: qs of chunk ch (both nibbles); 8 bytes a chunk:
+//         (d sc0, d sc1), (dmin m0, dmin m1)
 //   Q6_K  pieces 2 ch + h: ql; 4 + h: qh; 8 bytes a chunk: (d sc0, d sc1) of
-//         K half 0, of half 1
-//   Q8_0  (one chunk) pieces 2 h + {0, 1}: the codes of block 2 c + h; 4
-//         bytes a block: (d, d)
+//         its values 0 .. 15 of each sub-block, then of 16 .. 31
+//   Q8_0  (one chunk) pieces 2 h + b: the codes of block 2 c + b; 4 bytes a
+//         block: (d, d)
 template <int QT>
 struct WRow {
   static constexpr int kUnit = QT == kTypeQ8_0 ? 1 : 2;  // chunks
@@ -283,6 +286,13 @@ __device__ __forceinline__ void fetch_w(RawW<QT, NT> &w, rsrc_t Wr, int n0, int 
   }
 }
 
+// 16 bytes from a piece-aligned place p: the two K halves' 8 bytes of a piece
+// each (8-byte stores: one instruction, no more bank cycles than a 16-byte one).
+__device__ __forceinline__ void put_halves(uint8_t *p, u32x4 q) {
+  *reinterpret_cast<u32x2 *>(p) = u32x2{q.x, q.y};
+  *reinterpret_cast<u32x2 *>(p + 16) = u32x2{q.z, q.w};
+}
+
 // Scales: small integers become fp16 exactly under the magic 1024 (sc ^ 0x80
 // for Q6_K's signed ones), so each product is rounded once, as d * sc in
 // fp32 rounded to fp16 would be.
@@ -294,7 +304,7 @@ __device__ __forceinline__ void commit_w(uint8_t *rows, const RawW<QT, NT> &w, i
   if constexpr (QT == kTypeQ4_K) {
 #pragma unroll
     for (int i = 0; i < R::kCodes; ++i)
-      *reinterpret_cast<u32x4 *>(rows + (16 * i + (lane >> 2)) * L::kPitch + 16 * (lane & 3)) = w.q[i];
+      put_halves(rows + (16 * i + (lane >> 2)) * L::kPitch + 32 * ((lane >> 1) & 1) + 8 * (lane & 1), w.q[i]);
 #pragma unroll
     for (int i = 0; i < R::kHeads; ++i) {
       // get_scale_min_k4 (quant_common.cuh:83-94): sub-blocks 0..3 (un even)
@@ -320,17 +330,16 @@ __device__ __forceinline__ void commit_w(uint8_t *rows, const RawW<QT, NT> &w, i
   } else if constexpr (QT == kTypeQ6_K) {
 #pragma unroll
     for (int i = 0; i < 2 * NT; ++i)
-      *reinterpret_cast<u32x4 *>(rows + (16 * i + (lane >> 2)) * L::kPitch + 16 * (lane & 3)) = w.q[i];
+      put_halves(rows + (16 * i + (lane >> 2)) * L::kPitch + 32 * ((lane >> 1) & 1) + 8 * (lane & 1), w.q[i]);
 #pragma unroll
     for (int i = 0; i < NT; ++i)
-      *reinterpret_cast<u32x4 *>(rows + (32 * i + (lane >> 1)) * L::kPitch + 64 + 16 * (lane & 1)) =
-          w.q[2 * NT + i];
+      put_halves(rows + (32 * i + (lane >> 1)) * L::kPitch + 64 + 8 * (lane & 1), w.q[2 * NT + i]);
 #pragma unroll
     for (int i = 0; i < R::kHeads; ++i) {
       const h2 d = splat(h2f(w.d[i]));
       u32x4 o;
 #pragma unroll
-      for (int k = 0; k < 4; ++k) {  // chunk hf = k >> 1, K half h = k & 1: bytes 2 hf + h of both words
+      for (int k = 0; k < 4; ++k) {  // chunk hf = k >> 1, values 16 p .. with p = k & 1: bytes 2 hf + p of both words
         const uint32_t b = ((w.hd[i].x >> (8 * k)) & 0xFFu) | (((w.hd[i].y >> (8 * k)) & 0xFFu) << 16);
         o[k] = as_u32((as_h2((b ^ 0x00800080u) | mg) + splat(-1152.0f)) * d);
       }
@@ -345,10 +354,10 @@ __device__ __forceinline__ void commit_w(uint8_t *rows, const RawW<QT, NT> &w, i
       const uint32_t sh = lane & 1 ? 0 : 16;
       const u32x4 a = w.q[2 * i], b = w.q[2 * i + 1];
       auto cat = [&](uint32_t hi, uint32_t lo) { return __builtin_amdgcn_alignbit(hi, lo, sh); };
-      *reinterpret_cast<u32x4 *>(t + 32 * (lane & 1)) =
-          u32x4{cat(a.y, a.x), cat(a.z, a.y), cat(a.w, a.z), cat(b.x, a.w)};
-      *reinterpret_cast<u32x4 *>(t + 32 * (lane & 1) + 16) =
-          u32x4{cat(b.y, b.x), cat(b.z, b.y), cat(b.w, b.z), cat(w.d[i], b.w)};
+      *reinterpret_cast<u32x4 *>(t + 16 * (lane & 1)) =
+          u32x4{cat(a.y, a.x), cat(a.z, a.y), cat(b.y, b.x), cat(b.z, b.y)};
+      *reinterpret_cast<u32x4 *>(t + 32 + 16 * (lane & 1)) =
+          u32x4{cat(a.w, a.z), cat(b.x, a.w), cat(b.w, b.z), cat(w.d[i], b.w)};
       // d: the low half of the even block's first dword; the odd block's
       // follows the even one's codes (the high half of the lane before's last)
       const uint32_t before = dpp<0xA0>(0u, w.d[i]);  // quad_perm [0,0,2,2], in all lanes
@@ -359,7 +368,8 @@ __device__ __forceinline__ void commit_w(uint8_t *rows, const RawW<QT, NT> &w, i
 }
 
 // One lane's staged weights of a chunk: the 32 values that its K half h =
-// lane / 32 supplies to the chunk's four MFMAs, and their scales.
+// lane / 32 supplies to the chunk's four MFMAs, and their scales (d; n: Q4_K's
+// minima, Q6_K's scales of values 16 .. 31, Q8_0's second block).
 template <int QT>
 struct LaneW {
   u32x4 q, x;
@@ -378,11 +388,15 @@ __device__ __forceinline__ LaneW<QT> read_w(const uint8_t *row, int ch, int h) {
     w.q = *reinterpret_cast<const u32x4 *>(row + 16 * (2 * ch + h));
     const u32x4 x = *reinterpret_cast<const u32x4 *>(row + 64 + 16 * h);
     w.x = u32x4{x.x >> (2 * ch), x.y >> (2 * ch), x.z >> (2 * ch), x.w >> (2 * ch)};
-    w.d = as_h2(*reinterpret_cast<const uint32_t *>(row + L::kScale + 8 * ch + 4 * h));
+    const u32x2 s = *reinterpret_cast<const u32x2 *>(row + L::kScale + 8 * ch);
+    w.d = as_h2(s.x);
+    w.n = as_h2(s.y);
   } else {
     w.q = *reinterpret_cast<const u32x4 *>(row + 32 * h);
     w.x = *reinterpret_cast<const u32x4 *>(row + 32 * h + 16);
-    w.d = as_h2(*reinterpret_cast<const uint32_t *>(row + L::kScale + 4 * h));
+    const u32x2 s = *reinterpret_cast<const u32x2 *>(row + L::kScale);
+    w.d = as_h2(s.x);
+    w.n = as_h2(s.y);
   }
   return w;
 }
@@ -391,8 +405,9 @@ __device__ __forceinline__ LaneW<QT> read_w(const uint8_t *row, int ch, int h) {
 template <int QT>
 __device__ __forceinline__ h8 w_slot(const LaneW<QT> &w, int sl) {
   uint32_t o[4];
-  const h2 d = sl < 2 || QT == kTypeQ8_0 ? __builtin_shufflevector(w.d, w.d, 0, 0)
-                                         : __builtin_shufflevector(w.d, w.d, 1, 1);
+  const h2 ds = (QT == kTypeQ6_K && (sl & 1)) || (QT == kTypeQ8_0 && sl >= 2) ? w.n : w.d;
+  const h2 d = sl < 2 || QT == kTypeQ8_0 ? __builtin_shufflevector(ds, ds, 0, 0)
+                                         : __builtin_shufflevector(ds, ds, 1, 1);
   if constexpr (QT == kTypeQ4_K) {
     const h2 n = sl < 2 ? __builtin_shufflevector(w.n, w.n, 0, 0)
                         : __builtin_shufflevector(w.n, w.n, 1, 1);
@@ -426,10 +441,7 @@ __device__ __forceinline__ h8 w_slot(const LaneW<QT> &w, int sl) {
 
 // Activation group (8 values) that K half h supplies to slot sl: the
 // values the weights of that half and slot belong to.
-template <int QT>
-__device__ __forceinline__ int a_group(int sl, int h) {
-  return QT == kTypeQ8_0 ? 4 * h + sl : 4 * (sl >> 1) + 2 * h + (sl & 1);
-}
+__device__ __forceinline__ int a_group(int sl, int h) { return 2 * sl + h; }
 
 // C consecutive outputs (m, n ..) = v by the launch's epilogue: 16-byte
 // accesses where the row pitch allows (g.vec), single ones at ragged edges.
@@ -630,7 +642,7 @@ __global__ __launch_bounds__(64 * WN * KW, 2) void k_gemm_f16(const F16Args g) {
   };
   auto read_a = [&](h8 (&f)[MT], const _Float16 *sa, int sl) {
     // rows l32 + 32 i share swz(l32): period 16
-    const int ga = 8 * (a_group<QT>(sl, h) ^ swz(l32));
+    const int ga = 8 * (a_group(sl, h) ^ swz(l32));
 #pragma unroll
     for (int i = 0; i < MT; ++i)
       f[i] = *reinterpret_cast<const h8 *>(sa + (l32 + 32 * i) * kPitch + ga);
