@@ -431,7 +431,11 @@ int ifx_kernel_family(int quant_type, int M, int N, int K);
 /* Launch log of the calling thread.  ifx_launch_log_begin opens it: every
  * kernel that the entry points called afterwards on this thread launch is
  * recorded by instance name ("k_gemv<12,1,2,1,4,0,2>": kernel name and
- * template arguments as integers, ';'-separated, in launch order).  With
+ * template arguments as integers, ';'-separated, in launch order).  The
+ * prefill and int8 GEMMs, whose tile is planned per launch, add it in
+ * brackets: "k_gemm_f16<type,waves,fp16 out,1 atomic / 2 slots,fp16
+ * activations>[32-row tiles,32-column tiles,column waves,K waves,chunks a stage]"
+ * and "k_gemm_mfma<type,64-row tiles,fp16 out>[wave groups]".  With
  * dry_run != 0 nothing is launched (no HIP call is made, no pointer is
  * dereferenced; entry points return IFX_OK after validation), so the
  * dispatch of any shape can be inspected on a host without a GPU.

@@ -106,20 +106,23 @@ struct LaunchLog {
 thread_local LaunchLog g_log;
 }  // namespace
 
-bool note_launch(const char *kernel, std::initializer_list<int> targs) {
+bool note_launch(const char *kernel, std::initializer_list<int> targs,
+                 std::initializer_list<int> tile) {
   if (g_log.open) {
     if (!g_log.text.empty()) g_log.text += ';';
     g_log.text += kernel;
-    if (targs.size()) {
-      g_log.text += '<';
-      bool first = true;
-      for (int v : targs) {
-        if (!first) g_log.text += ',';
+    auto list = [](char open, std::initializer_list<int> vs, char close) {
+      if (!vs.size()) return;
+      char sep = open;
+      for (int v : vs) {
+        g_log.text += sep;
         g_log.text += std::to_string(v);
-        first = false;
+        sep = ',';
       }
-      g_log.text += '>';
-    }
+      g_log.text += close;
+    };
+    list('<', targs, '>');
+    list('[', tile, ']');
   }
   return !g_log.dry;
 }

@@ -785,9 +785,10 @@ hipError_t launch_tile(const F16Args &g, int grid, hipStream_t s) {
         reinterpret_cast<const void *>(fn), hipFuncAttributeMaxDynamicSharedMemorySize, T::kLds);
     if (attr != hipSuccess) return attr;
   }
-  // the log names the type, the waves, the epilogue and AH, not the tile
+  // type, waves, epilogue (fp16; 1 atomic, 2 slots) and AH, then the tile
   if (note_launch("k_gemm_f16", {QT, T::kThreads / 64, g.epi == kEpiF16,
-                                 g.epi == kEpiAtomic ? 1 : g.epi == kEpiSlot ? 2 : 0, AH}))
+                                 g.epi == kEpiAtomic ? 1 : g.epi == kEpiSlot ? 2 : 0, AH},
+                  {MT, NT, WN, KW, AU}))
     hipLaunchKernelGGL(fn, dim3(static_cast<unsigned>(grid)), dim3(T::kThreads), T::kLds, s, g);
   return last_error();
 }

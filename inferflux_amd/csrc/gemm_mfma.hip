@@ -490,8 +490,7 @@ __global__ __launch_bounds__(256 * KW, KW == 1 ? 2 : 4) void k_gemm_mfma(MfmaArg
 template <int QT, int S, bool F16OUT, int KW>
 static hipError_t launch_k(const MfmaArgs &g, dim3 grid, hipStream_t s) {
   const size_t shm = KW * sizeof(Smem<QT, S>);
-  // The log names the type, the tile and the output, not KW.
-  if (!note_launch("k_gemm_mfma", {QT, S, F16OUT})) return hipSuccess;
+  if (!note_launch("k_gemm_mfma", {QT, S, F16OUT}, {KW})) return hipSuccess;
   // The staged tiles can exceed the 64 KiB default; gfx950 has 160 KiB of LDS.
   // set once per kernel (function-local static: thread-safe)
   static const hipError_t attr = hipFuncSetAttribute(

@@ -75,7 +75,8 @@ inline const char *tuning_env(const char *name) {
 // integers) while a log is open on the calling thread, and skips the launch
 // itself in dry-run mode (ifx_launch_log_begin, include/ifx_qgemm.h), so the
 // dispatch can be inspected on a host without a GPU.
-bool note_launch(const char *kernel, std::initializer_list<int> targs);
+bool note_launch(const char *kernel, std::initializer_list<int> targs,
+                 std::initializer_list<int> tile = {});
 bool dry_run();
 // hipGetLastError / hipPeekAtLastError, or hipSuccess in dry-run mode.
 hipError_t last_error();

@@ -536,11 +536,13 @@ class launch_log:
     include/ifx_qgemm.h).  dry=True launches nothing: no HIP call is made, so
     the dispatch of any shape can be read on a host without a GPU (use fake
     non-null pointers then).  After the block, `.kernels` is the list of
-    instance names, e.g. ["k_gemv<12,1,2,1,4,0,2>"]."""
+    kernel names, e.g. ["k_gemv<12,1,2,1,4,0,2>"], and `.instances` the same with
+    the tile where a plan chooses one, e.g. "k_gemm_f16<12,8,0,0,0>[4,2,8,1,2]"."""
 
     def __init__(self, dry=False):
         self.dry = dry
         self.kernels = []
+        self.instances = []
 
     def __enter__(self):
         _lib.load().ifx_launch_log_begin(1 if self.dry else 0)
@@ -548,5 +550,6 @@ class launch_log:
 
     def __exit__(self, *exc):
         text = _lib.load().ifx_launch_log_end().decode()
-        self.kernels = text.split(";") if text else []
+        self.instances = text.split(";") if text else []
+        self.kernels = [k.split("[")[0] for k in self.instances]
         return False

@@ -22,21 +22,23 @@ def dev():
     return torch.device("cuda:0")
 
 
-# (M, N, K): the smallest tile and one past its edges, K of one chunk (Q8_0) or
-# one super-block, K ends inside a group of K waves, then sizes wide enough for
-# each larger tile (32 x 128, 64 x 128, 64 x 256, 96 x 256, 128 x 256, 128 x 512)
-SHAPES = [(33, 64, 256), (64, 65, 512), (96, 63, 768), (33, 8192, 256), (65, 8201, 1280),
+# (M, N, K): the smallest tile and one past its edges, K of one super-block, K
+# ends inside a group of K waves, then sizes wide enough for each larger tile
+# (32 x 128, 64 x 128, 64 x 256, 96 x 256, 128 x 256, 128 x 512).
+# test_prefill_splits.py checks which tiles these reach.
+SHAPES = [(33, 64, 256), (64, 65, 512), (96, 63, 768), (65, 8201, 1280), (257, 4100, 512),
           (100, 22016, 512), (191, 22017, 768), (256, 22016, 256), (385, 22020, 512),
           (513, 33000, 256)]
+# Q8_0 takes any K of whole 64-value chunks: one, and odd counts
+CASES = [(t, M, N, K) for t in (Q4_K, Q6_K) for M, N, K in SHAPES] + \
+    [(Q8_0, M, N, K - 64 * (M % 2) - 128 * (K > 256)) for M, N, K in SHAPES] + \
+    [(Q8_0, 35, 70, 64), (Q8_0, 300, 11009, 64)]
 
 
-@pytest.mark.parametrize("qtype", [Q4_K, Q6_K, Q8_0])
-@pytest.mark.parametrize("M,N,K", SHAPES)
+@pytest.mark.parametrize("qtype,M,N,K", CASES)
 def test_prefill_tiles(orc, dev, qtype, M, N, K):
     import torch
     from inferflux_amd import ops, synth
-    if qtype == Q8_0:
-        K -= 64 * (M % 2) + 128 * (K > 256)  # odd chunk counts too
     note(f"prefill tiles type={qtype} M={M} N={N} K={K}")
     w = synth.blocks(qtype, N, K, seed=N + K)
     a = orc.quantize_q8_1(synth.activations(M, K, seed=M + K, outlier_frac=0.01))
@@ -59,11 +61,18 @@ def test_prefill_tiles(orc, dev, qtype, M, N, K):
     check_rows(down(y16)[:, idx].astype(np.float64), ye, tol=2e-3)
 
 
-@pytest.mark.parametrize("qtype,M,Ns,K,f16", [
+# fp16 outputs do not split K; of the fp32 ones the first three do, into
+# outputs that the launch before clears
+GROUPED = [
+    (Q4_K, 130, (512, 64, 65), 2048, False), (Q6_K, 40, (1000, 33), 4096, False),
+    (Q8_0, 130, (300, 64, 65), 2048, False),
     (Q4_K, 130, (300, 64, 65), 512, False), (Q4_K, 600, (2048, 256, 256), 256, True),
-    (Q6_K, 40, (1000, 1), 1024, False), (Q8_0, 129, (77, 500, 31), 448, True),
-    (Q8_0, 300, (4097, 4096), 192, False),
-])
+    (Q6_K, 40, (1000, 1), 1024, False), (Q8_0, 129, (77, 500, 31), 768, True),
+    (Q8_0, 300, (4097, 4096), 256, False),
+]
+
+
+@pytest.mark.parametrize("qtype,M,Ns,K,f16", GROUPED)
 def test_prefill_grouped(orc, dev, qtype, M, Ns, K, f16):
     """Sibling projections in one launch: stored, and added to what is there."""
     import torch
@@ -75,6 +84,7 @@ def test_prefill_grouped(orc, dev, qtype, M, Ns, K, f16):
     dt = torch.float16 if f16 else torch.float32
     with ops.launch_log() as lg:
         ys = ops.qgemv_grouped(qtype, Ws, A, M, list(Ns), K, out_dtype=dt)
+    assert lg.kernels[-1].startswith("k_gemm_f16<"), lg.kernels
     assert [k for k in lg.kernels if k != "k_fill_zero"] == [lg.kernels[-1]]  # one GEMM launch
     base = [torch.full((M, n), 2.0, dtype=dt, device=dev) for n in Ns]
     ops.qgemv_grouped(qtype, Ws, A, M, list(Ns), K, outs=base, mode=ops.ACCUM)
@@ -88,3 +98,52 @@ def test_prefill_grouped(orc, dev, qtype, M, Ns, K, f16):
             tol = 2e-2
         assert np.all(np.abs(down(y).astype(np.float64) - ye) <= tol * np.maximum(bar, 1e-6) + (2e-3 * np.abs(ye) if f16 else 0))
         assert np.all(np.abs(down(b).astype(np.float64) - ye - 2.0) <= tol * np.maximum(bar, 1e-6) + (4e-3 * (np.abs(ye) + 2) if f16 else 0))
+
+
+# The fp16 copy of the activations (wide projections with a workspace), and
+# K splits of the wider tiles: added with atomics, or in order
+@pytest.mark.parametrize("qtype,M,N,K", [
+    (Q4_K, 96, 16387, 256), (Q4_K, 96, 18432, 1280), (Q4_K, 200, 27648, 512), (Q4_K, 100, 49152, 256),
+    (Q6_K, 33, 16384, 256), (Q6_K, 33, 18435, 768), (Q6_K, 66, 49152, 256), (Q6_K, 129, 49152, 256),
+    (Q8_0, 128, 16384, 320), (Q8_0, 128, 18432, 192), (Q8_0, 129, 22020, 64), (Q8_0, 129, 49152, 256),
+])
+def test_prefill_workspace(orc, dev, qtype, M, N, K):
+    import torch
+    from inferflux_amd import ops, synth
+    note(f"prefill workspace type={qtype} M={M} N={N} K={K}")
+    w = synth.blocks(qtype, N, K, seed=N + K)
+    a = orc.quantize_q8_1(synth.activations(M, K, seed=M + K, outlier_frac=0.01))
+    W, A = up(w, dev), up(a, dev)
+    ws = torch.empty(ops.prefill_workspace_bytes(qtype, M, N, K), dtype=torch.uint8, device=dev)
+    with ops.launch_log() as lg:
+        y = ops.qgemm_prefill_ws(qtype, W, A, M, N, K, ws)
+    assert lg.kernels[0] == "k_q8_1_to_f16" and lg.kernels[-1].endswith(",1>"), lg.kernels
+    assert torch.equal(y, ops.qgemm_prefill_kernel(qtype, W, A, M, N, K, ops.PREFILL_F16))
+    idx = np.unique(np.concatenate([[0, 31, N - 1], np.random.default_rng(N).choice(N, 96)]))
+    check_rows(down(y)[:, idx], orc.gemv_exact(qtype, w[idx], a, M, len(idx), K))
+
+
+@pytest.mark.parametrize("qtype,M,N,K", [
+    (Q4_K, 96, 1025, 5120), (Q4_K, 100, 2052, 13824), (Q6_K, 65, 1536, 8192), (Q6_K, 100, 1030, 13824),
+    (Q8_0, 129, 4100, 4160), (Q8_0, 128, 1027, 11008),
+])
+def test_prefill_wide_splits(orc, dev, qtype, M, N, K):
+    import torch
+    from inferflux_amd import ops, synth
+    note(f"prefill wide splits type={qtype} M={M} N={N} K={K}")
+    w = synth.blocks(qtype, N, K, seed=N + K)
+    a = orc.quantize_q8_1(synth.activations(M, K, seed=M + K, outlier_frac=0.01))
+    W, A = up(w, dev), up(a, dev)
+    idx = np.unique(np.concatenate([[0, N - 1], np.random.default_rng(N).choice(N, 96)]))
+    ye = orc.gemv_exact(qtype, w[idx], a, M, len(idx), K)
+    with ops.launch_log() as lg:
+        y = ops.qgemm_prefill_kernel(qtype, W, A, M, N, K, ops.PREFILL_F16)
+    assert lg.kernels[0] == "k_fill_zero" and ",1,0>" in lg.kernels[1], lg.kernels
+    check_rows(down(y)[:, idx], ye)
+    ws = torch.empty(ops.prefill_ordered_workspace_bytes(qtype, M, N, K), dtype=torch.uint8,
+                     device=dev)
+    y = torch.full((M, N), 1.0, device=dev)
+    with ops.launch_log() as lg:
+        ops.qgemm_prefill_ordered(qtype, W, A, M, N, K, ws, out=y, mode=ops.ACCUM)
+    assert ",2,0>" in lg.kernels[0] and lg.kernels[1] == "k_split_sum", lg.kernels
+    check_rows(down(y)[:, idx], ye + 1.0)

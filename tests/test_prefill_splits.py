@@ -1,7 +1,9 @@
-"""K splits of the fp16 prefill GEMM: the ordered entry asks for no more
-workspace than the documented line (a grid of 256 x 256 tiles, 512 values of
+"""K splits and tiles of the fp16 prefill GEMM, planned on the host: the ordered
+entry asks for no more workspace than the documented line (a grid of 256 x 256 tiles, 512 values of
 K a split), so a buffer sized for a shape once stays large enough, and a
-shape that never split still runs without one."""
+shape that never split still runs without one; and the GPU tests' shapes reach
+every tile."""
+import ctypes
 import itertools
 
 import pytest
@@ -31,3 +33,40 @@ def test_ordered_workspace_within_the_line(qt):
         line = _line(M, N, K)  # the slots follow the fp16 copy, 256-byte aligned
         assert need <= (-(-copy // 256) * 256 + line if line else copy), (M, N, K)
         assert ops.prefill_ordered_workspace_bytes(qt, M, N, K, torch.float16) <= copy
+
+
+def _instances(call, qt, M, N, K, *more):
+    """Instances that an entry of one projection would launch."""
+    p = [ctypes.c_void_p(0x100000 * (i + 1)) for i in range(4)]
+    from inferflux_amd import _lib
+    with ops.launch_log(dry=True) as lg:
+        rc = getattr(_lib.load(), call)(qt, p[0], p[1], p[2], ops.OUT_F32, ops.STORE, None, M, N, K,
+                                        *[p[3] if m == "ws" else m for m in more], None)
+    assert rc == 0
+    return lg.instances
+
+
+# 32-row and 32-column MFMA tiles, waves along the columns, waves along K
+TILES = {(4, 2, 8, 1), (4, 2, 4, 2), (3, 2, 4, 2), (2, 2, 4, 2), (2, 2, 2, 4), (1, 2, 2, 4),
+         (1, 2, 1, 8)}
+
+
+def _tile(name):
+    return tuple(int(v) for v in name.split("[")[1][:-1].split(","))[:4]
+
+
+@pytest.mark.parametrize("qt", [Q4_K, Q6_K, Q8_0])
+def test_gpu_shapes_reach_every_tile(qt):
+    from tests.test_gpu_prefill_tiles import CASES
+    got = {_tile(_instances("ifx_qgemm_prefill_kernel", qt, M, N, K, ops.PREFILL_F16, 0)[-1])
+           for t, M, N, K in CASES if t == qt}
+    assert got == TILES
+
+
+def test_int8_gpu_shapes_reach_every_group_count():
+    from tests.test_gpu_mid_batch import CASES
+    for qt in (Q4_K, Q8_0):
+        got = {k for t, M, Ns, K in CASES if t == qt
+               for k in _instances("ifx_qgemm_prefill_kernel", qt, M, Ns[0], K, ops.PREFILL_INT8, 0)}
+        want = {f"k_gemm_mfma<{qt},1,0>[{kw}]" for kw in (1, 2, 4)}
+        assert want <= got, got
