@@ -793,8 +793,9 @@ hipError_t launch_tile(const F16Args &g, int grid, hipStream_t s) {
   return last_error();
 }
 
-// The tiles a launch can take (kF16Tiles in gemm_f16.hip).  All have eight waves;
-// those with fewer along n split the stage's K range.
+// The tiles a launch can take (kF16Tiles in gemm_f16.hip).  All but the last have
+// eight waves; those with fewer along n split the stage's K range.  The last, on
+// four waves, sums K in order (kOrderedTile).
 template <int QT, bool AH>
 hipError_t launch_by_tile(int tile, const F16Args &g, int grid, hipStream_t s) {
   switch (tile) {
@@ -804,7 +805,10 @@ hipError_t launch_by_tile(int tile, const F16Args &g, int grid, hipStream_t s) {
   case 3: return launch_tile<QT, AH, 2, 2, 4, 2, QT == kTypeQ8_0 || AH ? 1 : 2>(g, grid, s);
   case 4: return launch_tile<QT, AH, 2, 2, 2, 4, 1>(g, grid, s);
   case 5: return launch_tile<QT, AH, 1, 2, 2, 4, 1>(g, grid, s);
-  default: return launch_tile<QT, AH, 1, 2, 1, 8, 1>(g, grid, s);
+  case 6: return launch_tile<QT, AH, 1, 2, 1, 8, 1>(g, grid, s);
+  default:
+    if constexpr (QT == kTypeQ8_0 || AH) return hipErrorInvalidValue;  // not planned
+    else return launch_tile<QT, AH, 2, 1, 4, 1, 2>(g, grid, s);
   }
 }
 

@@ -86,8 +86,23 @@ constexpr TileInfo kF16Tiles[] = {
     {64, 128, 4, {{4.9f, 4.8f, 1.1f}, {4.7f, 6.8f, 1.2f}, {5.8f, 6.0f, 0.8f}}},
     {32, 128, 4, {{3.2f, 3.9f, 0.5f}, {3.8f, 5.6f, 0.4f}, {3.8f, 5.3f, 0.7f}}},
     {32, 64, 8, {{3.3f, 2.1f, 0.4f}, {4.3f, 3.1f, 0.5f}, {4.2f, 2.7f, 0.3f}}},
+    {64, 128, 1, {{3.0f, 7.2f, 0.0f}, {3.4f, 8.1f, 0.0f}, {}}},
 };
 constexpr int kNTiles = sizeof(kF16Tiles) / sizeof(kF16Tiles[0]);
+
+// Long prompts' narrow projections in order: a launch of kOrderedM rows or more
+// whose sums no split along K divides (K-quants, less than the fp16 copy's
+// columns) can take the last tile, 64 x 128 without K waves, and takes a tile
+// with K waves only where that is slower by more than kOrderedCost.  K and V of
+// a 14B layer at M = 1999 (Q4_K 1999 x 1024 x 5120) take 46 us so and 38 with K
+// waves, under 1 % of the layer, and all its outputs have the bits of a sum
+// over K in steps of 16 (Q, O, gate, up and down take 128 x 512).  K and V of a
+// 3B model (256 columns, 20 us against 11), wider projections on the 256-column tiles
+// (1024 x 5120 x 5120, 91 against 74), Q8_0 (59 against 45 at 1999 x 1024 x 5120) and
+// shorter prompts (512 x 1024 x 5120, 40 against 19) keep the K waves.
+constexpr int kOrderedTile = kNTiles - 1;
+constexpr int kOrderedM = 1024, kOrderedN = 16384;
+constexpr float kOrderedCost = 1.25f;
 
 struct Plan {
   int tile, m_tiles, n_tiles, splits, spw;
@@ -127,10 +142,11 @@ Plan f16_plan(int qt, bool f16, int count, const int *N, int M, int K, int split
   const int cap = f16 ? 1 : max_splits(count, N, M, K);
   int64_t n_sum = 0;
   for (int i = 0; i < count; ++i) n_sum += N[i];
+  const bool in_order = qt != kTypeQ8_0 && M >= kOrderedM && n_sum < kOrderedN && cap == 1;
   Plan best{};
   float best_cost = 0.0f;
   for (int ti = 0; ti < kNTiles; ++ti) {
-    if (forced >= 0 && ti != forced) continue;
+    if (forced >= 0 ? ti != forced : ti == kOrderedTile && !in_order) continue;
     const TileInfo &t = kF16Tiles[ti];
     Plan p{};
     p.tile = ti;
@@ -151,6 +167,7 @@ Plan f16_plan(int qt, bool f16, int count, const int *N, int M, int K, int split
       const float w = static_cast<float>(wg * p.splits) / 256.0f, rounds = std::ceil(w);
       const float k = static_cast<float>(std::min(p.spw * kc, nch) * kBK) / 1024.0f;
       float cost = rounds * (t.cost[ty].a + t.cost[ty].b * k) + t.cost[ty].c * w * k;
+      if (in_order && t.kw > 1) cost *= kOrderedCost;
       if (p.splits > 1) cost += 4.0f + 2e-6f * p.splits * static_cast<float>(n_sum) * M;
       if (best_cost == 0.0f || cost < best_cost) best_cost = cost, best = p;
     }

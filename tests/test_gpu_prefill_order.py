@@ -45,3 +45,18 @@ def test_sums_run_over_k_in_order(orc, dev, qtype, K, crc32, crc16):
     y = down(ops.qgemm_prefill_kernel(qtype, W, A, M, N, K, ops.PREFILL_F16,
                                       out_dtype=torch.float16))
     assert zlib.crc32(y.tobytes()) == crc16
+
+
+# Long prompts' narrow projections (K and V), fp16
+@pytest.mark.parametrize("qtype,N,K,crc", [
+    (Q4_K, 1024, 512, 0x567f4461), (Q4_K, 1024, 5120, 0x2351e596),
+    (Q6_K, 1024, 512, 0xdf22c5d3), (Q6_K, 1024, 2560, 0x7367ad3b)])
+def test_long_prompt_sums_run_over_k_in_order(orc, dev, qtype, N, K, crc):
+    import torch
+    from inferflux_amd import ops, synth
+    note(f"prefill order type={qtype} M=1999 N={N} K={K}")
+    w = synth.blocks(qtype, N, K, seed=5)
+    a = orc.quantize_q8_1(synth.activations(1999, K, seed=6, outlier_frac=0.01))
+    y = ops.qgemm_prefill_kernel(qtype, up(w, dev), up(a, dev), 1999, N, K, ops.PREFILL_F16,
+                                 out_dtype=torch.float16)
+    assert zlib.crc32(down(y).tobytes()) == crc

@@ -29,8 +29,10 @@ def dev():
 SHAPES = [(33, 64, 256), (64, 65, 512), (96, 63, 768), (65, 8201, 1280), (257, 4100, 512),
           (100, 22016, 512), (191, 22017, 768), (256, 22016, 256), (385, 22020, 512),
           (513, 33000, 256)]
+# and a long prompt's 64 x 128 tile in order (Q4_K, Q6_K).
+LONG = (1025, 1030, 512)
 # Q8_0 takes any K of whole 64-value chunks: one, and odd counts
-CASES = [(t, M, N, K) for t in (Q4_K, Q6_K) for M, N, K in SHAPES] + \
+CASES = [(t, M, N, K) for t in (Q4_K, Q6_K) for M, N, K in SHAPES + [LONG]] + \
     [(Q8_0, M, N, K - 64 * (M % 2) - 128 * (K > 256)) for M, N, K in SHAPES] + \
     [(Q8_0, 35, 70, 64), (Q8_0, 300, 11009, 64)]
 

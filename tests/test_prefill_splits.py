@@ -35,12 +35,12 @@ def test_ordered_workspace_within_the_line(qt):
         assert ops.prefill_ordered_workspace_bytes(qt, M, N, K, torch.float16) <= copy
 
 
-def _instances(call, qt, M, N, K, *more):
+def _instances(call, qt, M, N, K, *more, f16=False):
     """Instances that an entry of one projection would launch."""
     p = [ctypes.c_void_p(0x100000 * (i + 1)) for i in range(4)]
     from inferflux_amd import _lib
     with ops.launch_log(dry=True) as lg:
-        rc = getattr(_lib.load(), call)(qt, p[0], p[1], p[2], ops.OUT_F32, ops.STORE, None, M, N, K,
+        rc = getattr(_lib.load(), call)(qt, p[0], p[1], p[2], ops.OUT_F16 if f16 else ops.OUT_F32, ops.STORE, None, M, N, K,
                                         *[p[3] if m == "ws" else m for m in more], None)
     assert rc == 0
     return lg.instances
@@ -49,6 +49,7 @@ def _instances(call, qt, M, N, K, *more):
 # 32-row and 32-column MFMA tiles, waves along the columns, waves along K
 TILES = {(4, 2, 8, 1), (4, 2, 4, 2), (3, 2, 4, 2), (2, 2, 4, 2), (2, 2, 2, 4), (1, 2, 2, 4),
          (1, 2, 1, 8)}
+ORDERED = (2, 1, 4, 1)  # Q4_K, Q6_K
 
 
 def _tile(name):
@@ -60,7 +61,23 @@ def test_gpu_shapes_reach_every_tile(qt):
     from tests.test_gpu_prefill_tiles import CASES
     got = {_tile(_instances("ifx_qgemm_prefill_kernel", qt, M, N, K, ops.PREFILL_F16, 0)[-1])
            for t, M, N, K in CASES if t == qt}
-    assert got == TILES
+    assert got == (TILES if qt == Q8_0 else TILES | {ORDERED})
+
+
+@pytest.mark.parametrize("qt", [Q4_K, Q6_K])
+@pytest.mark.parametrize("M,N,K", [(1999, 1024, 5120), (2048, 1024, 5120), (1025, 1030, 512),
+                                   (1999, 5120, 5120), (1999, 13824, 5120)])
+def test_long_prompts_sum_in_order(qt, M, N, K):
+    """fp16 outputs of a long prompt's layer: no waves along K."""
+    call = _instances("ifx_qgemm_prefill_kernel", qt, M, N, K, ops.PREFILL_F16, 0, f16=True)
+    assert len(call) == 1 and _tile(call[0])[3] == 1, call
+
+
+@pytest.mark.parametrize("qt,M,N,K", [(Q4_K, 1023, 1024, 5120), (Q4_K, 1999, 256, 2048),
+                                      (Q6_K, 1024, 5120, 5120), (Q8_0, 1999, 1024, 5120)])
+def test_other_launches_keep_the_k_waves(qt, M, N, K):
+    call = _instances("ifx_qgemm_prefill_kernel", qt, M, N, K, ops.PREFILL_F16, 0, f16=True)
+    assert _tile(call[0])[3] > 1, call
 
 
 def test_int8_gpu_shapes_reach_every_group_count():
