@@ -91,17 +91,17 @@ constexpr TileInfo kF16Tiles[] = {
 constexpr int kNTiles = sizeof(kF16Tiles) / sizeof(kF16Tiles[0]);
 
 // Long prompts' narrow projections in order: a launch of kOrderedM rows or more
-// whose sums no split along K divides (K-quants, less than the fp16 copy's
-// columns) can take the last tile, 64 x 128 without K waves, and takes a tile
+// whose sums no split along K divides (K-quants, less than kOrderedN columns in
+// all) can take the last tile, 64 x 128 without K waves, and takes a tile
 // with K waves only where that is slower by more than kOrderedCost.  K and V of
 // a 14B layer at M = 1999 (Q4_K 1999 x 1024 x 5120) take 46 us so and 38 with K
 // waves, under 1 % of the layer, and all its outputs have the bits of a sum
 // over K in steps of 16 (Q, O, gate, up and down take 128 x 512).  K and V of a
-// 3B model (256 columns, 20 us against 11), wider projections on the 256-column tiles
-// (1024 x 5120 x 5120, 91 against 74), Q8_0 (59 against 45 at 1999 x 1024 x 5120) and
+// 3B model (256 columns, 20 us against 11), wider projections where the plan takes a
+// tile with K waves (1024 x 5120 x 5120, 91 against 74), Q8_0 (59 against 45 at 1999 x 1024 x 5120) and
 // shorter prompts (512 x 1024 x 5120, 40 against 19) keep the K waves.
 constexpr int kOrderedTile = kNTiles - 1;
-constexpr int kOrderedM = 1024, kOrderedN = 16384;
+constexpr int kOrderedM = 1024, kOrderedN = 2048;
 constexpr float kOrderedCost = 1.25f;
 
 struct Plan {
