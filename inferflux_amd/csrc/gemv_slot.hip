@@ -117,12 +117,6 @@ __device__ __forceinline__ uint32_t q6_codes(uint32_t l4, uint32_t u2) {
   return __builtin_amdgcn_perm(0u, 0x1000F0E0u, u2) | l4;
 }
 
-__device__ __forceinline__ void wave_sync() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 // TL: the tiled layout (ifx_common.h), voff = 16 * (lane % 32) and sb_off
 // the tile's byte offset.
 template <int QT, bool TL = false>

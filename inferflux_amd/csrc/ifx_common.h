@@ -320,6 +320,15 @@ __device__ __forceinline__ float ld_dev(const float *p) {
   return __hip_atomic_load(const_cast<float *>(p), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
+// Between LDS accesses through which the lanes of one wave exchange data: the
+// hardware keeps a wave's LDS operations in order, this keeps the compiler
+// from moving one past another.  No instruction.
+__device__ __forceinline__ void wave_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // Ordered K-split reduction (the workspace entry points): every workgroup of
 // a split tile stores its fp32 partial sums to its own workspace slot with
 // st_dev, each wave waits for its stores (wait_own_memory), and the

@@ -209,12 +209,6 @@ __device__ __forceinline__ void commit(WaveLds<QT, MT> &L, const Chunks<QT, MT> 
   }
 }
 
-__device__ __forceinline__ void wave_sync() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 // LDS -> MFMA operands of this lane (weight row l16, K chunk q).
 template <int QT, int MT>
 __device__ __forceinline__ void read_w(WRegs<QT> &w, const WaveLds<QT, MT> &L, int l16, int q,
