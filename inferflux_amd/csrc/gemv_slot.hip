@@ -243,11 +243,16 @@ __device__ __forceinline__ i32x4 w_operand(const WSb<QT> &w, int j) {
 
 }  // namespace
 
-// NP: projections per workgroup (2 for the fused gate/up/SiLU launch).
-// Whether a launch stages raw rows (16 waves of Q6_K areas would pass 64 KB).
+// Whether a launch stages raw rows (the fused one with 16 waves does not: its
+// Q6_K areas alone take 112 KB, and it runs on request only).  Eight waves of
+// Q6_K areas pass 64 KB with the tables and sums (KW = 8, or the fused launch
+// with KW = 4: 67 and 68 KB, two workgroups a CU) and gain all the same: us
+// without and with, 1024 x 5120 at M = 8 12.2 -> 9.2, 5120 x 5120 13.2 -> 12.1, fused
+// 11008 x 2048 19.4 -> 18.6, 2048 x 6144 26.3 -> 21.3.
 template <int KW, bool SW, bool TL>
 constexpr bool slot_staged() { return !TL && !(SW && KW == 8); }
 
+// NP: projections per workgroup (2 for the fused gate/up/SiLU launch).
 template <int QT, int MP, int KW, bool SW, bool TL>
 constexpr int slot_lds_bytes() {
   constexpr int NP = SW ? 2 : 1;
@@ -664,9 +669,25 @@ void choose_slot_work(int blocks, int nsb, bool no_split, int &kw, int &ks) {
   ks = no_split ? 1 : max(1, min(ks, nsb / kw));
 }
 
+// Allows an instance's dynamic LDS where it is above the 64 KB default, once
+// (a function-local static: thread-safe).  A failure stays set for the launch's
+// hipGetLastError.
+template <int QT, int MP, int KW, bool F16OUT, int SPLIT, bool SW, bool TL>
+void slot_allow_lds() {
+  constexpr int lds = slot_lds_bytes<QT, MP, KW, SW, TL>();
+  if constexpr (lds > 65536) {
+    if (dry_run()) return;
+    static const hipError_t attr = hipFuncSetAttribute(
+        reinterpret_cast<const void *>(&k_gemv_slot<QT, MP, KW, F16OUT, SPLIT, SW, TL>),
+        hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+    (void)attr;
+  }
+}
+
 template <int QT, int MP, int KW, bool F16OUT, int SPLIT, bool TL>
 void slot_launch(const SlotArgs &args, int blocks, int ks, hipStream_t s) {
   constexpr int lds = slot_lds_bytes<QT, MP, KW, false, TL>();
+  slot_allow_lds<QT, MP, KW, F16OUT, SPLIT, false, TL>();
   if constexpr (TL)
     IFX_LAUNCH(k_gemv_slot, (QT, MP, KW, F16OUT, SPLIT, false, true), dim3(blocks, ks),
                dim3(64 * KW), lds, s, args);
@@ -734,6 +755,8 @@ template <int QT, int MP, int KW, bool TL>
 void slot_swiglu_launch(const SlotArgs &args, bool f16h, hipStream_t s) {
   constexpr int lds = slot_lds_bytes<QT, MP, KW, true, TL>();
   const dim3 grid(args.seg[0].N / 32);
+  if (f16h) slot_allow_lds<QT, MP, KW, true, false, true, TL>();
+  else slot_allow_lds<QT, MP, KW, false, false, true, TL>();
   if constexpr (TL) {
     if (f16h) IFX_LAUNCH(k_gemv_slot, (QT, MP, KW, true, false, true, true), grid, dim3(128 * KW), lds, s, args);
     else IFX_LAUNCH(k_gemv_slot, (QT, MP, KW, false, false, true, true), grid, dim3(128 * KW), lds, s, args);

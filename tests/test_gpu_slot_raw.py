@@ -24,6 +24,7 @@ def dev():
 @pytest.mark.parametrize("qtype,M,N,K", [
     (Q4_K, 4, 1, 256), (Q4_K, 8, 33, 2048), (Q4_K, 5, 8223, 512), (Q6_K, 5, 8192, 256),
     (Q6_K, 8, 8225, 768), (Q4_K, 6, 63, 2304), (Q6_K, 7, 31, 1024),
+    (Q6_K, 8, 1000, 2048), (Q6_K, 4, 33, 6144),  # eight waves: LDS past 64 KB
 ])
 def test_slot_raw_rows(orc, dev, qtype, M, N, K):
     from inferflux_amd import ops, synth
