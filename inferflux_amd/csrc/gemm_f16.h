@@ -604,7 +604,7 @@ __global__ __launch_bounds__(64 * WN * KW, 2) void k_gemm_f16(const F16Args g) {
     for (int u = 0; u < T::kAPt; ++u) {
       const int it = tid + T::kThreads * u;
       const int row = it / (2 * T::KC), c = item_chunk(x, it);
-      // (a chunk past K reads the next row's blocks, or past the end: zeroed below)
+      // (a chunk past K reads zeros, past every tensor)
       if (T::kAItems % T::kThreads == 0 || it < T::kAItems)
         fetch_a<QT, AH>(ra[u], Ar, c < nch ? min(m0 + row, M - 1) * a_row : kOobOffset, c < nch ? c : 0,
                         it & 1);

@@ -238,8 +238,8 @@ bool gemm_f16_fits(int qtype, int K) {
   return false;
 }
 
-// Bytes of the fp16 activation copy the GEMM can use (M x K halves), or 0
-// when it would not fit the kernel's 32-bit buffer offsets.
+// Bytes of the fp16 activation copy (M x K halves), or 0 when they would not fit
+// 32 bits.  Part of the interface; launches use a copy below kMaxBufferBytes only.
 int64_t gemm_f16_workspace_bytes(int M, int K) {
   const int64_t b = static_cast<int64_t>(M) * K * 2;
   return b < (int64_t{1} << 32) ? b : 0;
@@ -264,7 +264,9 @@ hipError_t launch_gemm_f16_grouped(int qtype, int count, const void *const *W, c
                                    hipStream_t stream, float *slots) {
   const uint8_t *a = static_cast<const uint8_t *>(A);
   if (!gemm_f16_fits(qtype, K)) return hipErrorInvalidValue;
-  if (A16 && gemm_f16_workspace_bytes(M, K) == 0) A16 = nullptr;
+  // chunks past K read zeros at kOobOffset, which has to lie past the copy
+  const uint64_t copy = gemm_f16_workspace_bytes(M, K);
+  if (copy == 0 || copy >= kMaxBufferBytes) A16 = nullptr;
   return launch_qt(qtype, count, W, a, A16, Y, N, bias, f16, M, K, mode, splits_req, slots, stream);
 }
 

@@ -80,6 +80,19 @@ def test_other_launches_keep_the_k_waves(qt, M, N, K):
     assert _tile(call[0])[3] > 1, call
 
 
+@pytest.mark.parametrize("qt", [Q4_K, Q6_K, Q8_0])
+def test_copy_ends_below_the_zero_offset(qt):
+    """Chunks past K read zeros at byte 0xF0000000, so no fp16 copy reaches it."""
+    N, K = 16384, 27648
+    for M, copied in ((72810, 1), (72817, 1), (72819, 0), (72900, 0), (77000, 0)):
+        assert (2 * M * K < 0xF0000000) == bool(copied)
+        nbytes = ops.prefill_workspace_bytes(qt, M, N, K)
+        assert nbytes == 2 * M * K  # what a caller hands over does not change
+        call = _instances("ifx_qgemm_prefill_ws", qt, M, N, K, "ws", nbytes)
+        assert call[-1].split("[")[0].endswith(f",{copied}>"), call
+        assert ("k_q8_1_to_f16" in call) == bool(copied)
+
+
 def test_int8_gpu_shapes_reach_every_group_count():
     from tests.test_gpu_mid_batch import CASES
     for qt in (Q4_K, Q8_0):
