@@ -783,6 +783,7 @@ __global__ __launch_bounds__(64 * WN * KW, 2) void k_gemm_f16(const F16Args g) {
   pass(std::integral_constant<int, 0>{});
   pass(std::integral_constant<int, T::PI>{});
   pass(std::integral_constant<int, 2 * T::PI>{});
+  pass(std::integral_constant<int, 3 * T::PI>{});
 }
 
 // Tile of a launch by index (f16_plan).
@@ -805,19 +806,38 @@ hipError_t launch_tile(const F16Args &g, int grid, hipStream_t s) {
 
 // The tiles a launch can take (kF16Tiles in gemm_f16.hip).  All but the last have
 // eight waves; those with fewer along n split the stage's K range.  The last, on
-// four waves, sums K in order (kOrderedTile).
+// four waves, sums K in order (kOrderedTile).  The largest is 128 x 512 for Q4_K
+// and 256 x 256 for Q6_K and Q8_0, where a weight is then converted once for 256
+// rows, not 128.  us on 128 x 512 / on 256 x 256, x 27648 x 5120 with the fp16 copy at
+// M = 384, 512, 1999, and 1999 x 13824 x 5120 without:
+//   Q8_0  185 / 150   184 / 155   720 / 628   355 / 335
+//   Q6_K  196 / 170   197 / 182   768 / 732   384 / 351
+//   Q4_K  135 / 146   153 / 153   598 / 624   297 / 316
+// Q6_K's 128 x 256 has its waves along n, too: with two K waves it needed more
+// registers than there are (four spilled with the fp16 copy) and took, with
+// the copy, 126 us at 256 x 27648 x 5120 (110 now), without 53 at 512 x 11008 x 2048 (48).
 template <int QT, bool AH>
 hipError_t launch_by_tile(int tile, const F16Args &g, int grid, hipStream_t s) {
   switch (tile) {
-  case 0: return launch_tile<QT, AH, 4, 2, 8, 1, QT == kTypeQ4_K ? 2 : 1>(g, grid, s);
-  case 1: return launch_tile<QT, AH, 4, 2, 4, 2, 1>(g, grid, s);
+  case 0:
+    if constexpr (QT != kTypeQ4_K) return hipErrorInvalidValue;  // not planned
+    else return launch_tile<QT, AH, 4, 2, 8, 1, 2>(g, grid, s);
+  case 1:
+    if constexpr (QT == kTypeQ6_K) return hipErrorInvalidValue;
+    else return launch_tile<QT, AH, 4, 2, 4, 2, 1>(g, grid, s);
   case 2: return launch_tile<QT, AH, 3, 2, 4, 2, 1>(g, grid, s);
   case 3: return launch_tile<QT, AH, 2, 2, 4, 2, QT == kTypeQ8_0 || AH ? 1 : 2>(g, grid, s);
   case 4: return launch_tile<QT, AH, 2, 2, 2, 4, 1>(g, grid, s);
   case 5: return launch_tile<QT, AH, 1, 2, 2, 4, 1>(g, grid, s);
   case 6: return launch_tile<QT, AH, 1, 2, 1, 8, 1>(g, grid, s);
+  case 7:
+    if constexpr (QT != kTypeQ6_K) return hipErrorInvalidValue;
+    else return launch_tile<QT, AH, 4, 1, 8, 1, 2>(g, grid, s);
+  case 8:
+    if constexpr (QT == kTypeQ4_K) return hipErrorInvalidValue;
+    else return launch_tile<QT, AH, 8, 1, 8, 1, 1>(g, grid, s);
   default:
-    if constexpr (QT == kTypeQ8_0 || AH) return hipErrorInvalidValue;  // not planned
+    if constexpr (QT == kTypeQ8_0 || AH) return hipErrorInvalidValue;
     else return launch_tile<QT, AH, 2, 1, 4, 1, 2>(g, grid, s);
   }
 }

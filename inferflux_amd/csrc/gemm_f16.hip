@@ -79,13 +79,15 @@ struct TileInfo {
   } cost[3];
 };
 constexpr TileInfo kF16Tiles[] = {
-    {128, 512, 1, {{17.0f, 19.4f, 7.0f}, {15.5f, 29.8f, 6.1f}, {16.5f, 26.2f, 7.3f}}},
-    {128, 256, 2, {{9.6f, 11.9f, 4.6f}, {11.0f, 14.9f, 4.5f}, {9.9f, 17.0f, 3.9f}}},
+    {128, 512, 1, {{17.0f, 19.4f, 7.0f}, {}, {}}},
+    {128, 256, 2, {{9.6f, 11.9f, 4.6f}, {}, {9.9f, 17.0f, 3.9f}}},
     {96, 256, 2, {{9.6f, 9.0f, 3.6f}, {8.2f, 14.7f, 3.2f}, {11.1f, 11.2f, 3.7f}}},
     {64, 256, 2, {{7.1f, 7.4f, 2.1f}, {7.5f, 11.9f, 1.7f}, {8.1f, 11.8f, 1.3f}}},
     {64, 128, 4, {{4.9f, 4.8f, 1.1f}, {4.7f, 6.8f, 1.2f}, {5.8f, 6.0f, 0.8f}}},
     {32, 128, 4, {{3.2f, 3.9f, 0.5f}, {3.8f, 5.6f, 0.4f}, {3.8f, 5.3f, 0.7f}}},
     {32, 64, 8, {{3.3f, 2.1f, 0.4f}, {4.3f, 3.1f, 0.5f}, {4.2f, 2.7f, 0.3f}}},
+    {128, 256, 1, {{}, {10.4f, 14.1f, 4.2f}, {}}},
+    {256, 256, 1, {{}, {14.0f, 26.8f, 5.5f}, {14.9f, 24.0f, 6.9f}}},
     {64, 128, 1, {{3.0f, 7.2f, 0.0f}, {3.4f, 8.1f, 0.0f}, {}}},
 };
 constexpr int kNTiles = sizeof(kF16Tiles) / sizeof(kF16Tiles[0]);
@@ -96,10 +98,11 @@ constexpr int kNTiles = sizeof(kF16Tiles) / sizeof(kF16Tiles[0]);
 // with K waves only where that is slower by more than kOrderedCost.  K and V of
 // a 14B layer at M = 1999 (Q4_K 1999 x 1024 x 5120) take 46 us so and 38 with K
 // waves, under 1 % of the layer, and all its outputs have the bits of a sum
-// over K in steps of 16 (Q, O, gate, up and down take 128 x 512).  K and V of a
+// over K in steps of 16 (Q, O, gate and up take 128 x 512, down 256 x 256).  K and V of a
 // 3B model (256 columns, 20 us against 11), wider projections where the plan takes a
-// tile with K waves (1024 x 5120 x 5120, 91 against 74), Q8_0 (59 against 45 at 1999 x 1024 x 5120) and
-// shorter prompts (512 x 1024 x 5120, 40 against 19) keep the K waves.
+// tile with K waves (1024 x 5120 x 5120, 91 against 74), Q8_0 (59 against 45 at
+// 1999 x 1024 x 5120) and shorter prompts (512 x 1024 x 5120, 40 against 19) keep
+// the K waves.
 constexpr int kOrderedTile = kNTiles - 1;
 constexpr int kOrderedM = 1024, kOrderedN = 2048;
 constexpr float kOrderedCost = 1.25f;
@@ -148,6 +151,7 @@ Plan f16_plan(int qt, bool f16, int count, const int *N, int M, int K, int split
   for (int ti = 0; ti < kNTiles; ++ti) {
     if (forced >= 0 ? ti != forced : ti == kOrderedTile && !in_order) continue;
     const TileInfo &t = kF16Tiles[ti];
+    if (t.cost[ty].b == 0.0f) continue;  // not a tile of this type
     Plan p{};
     p.tile = ti;
     p.m_tiles = (M + t.bm - 1) / t.bm;

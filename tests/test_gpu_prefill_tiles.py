@@ -1,5 +1,5 @@
-"""The fp16 prefill GEMM over the tile shapes its plan chooses from (32 x 64
-to 128 x 512): sizes at the edges of a tile and one past them, ragged K ends
+"""The fp16 prefill GEMM over the tile shapes its plan chooses from (32 x 64 to
+128 x 512 and 256 x 256): sizes at the edges of a tile and one past them, ragged K ends
 (K of one chunk, K groups that one wave's share ends inside), rows that do
 not start on 16 bytes, and projections that share a launch.  Checked against
 the fp64 oracle at 1e-3 * ||y_row||_2 (fp16 outputs 2e-3), the bar of the other
@@ -24,7 +24,7 @@ def dev():
 
 # (M, N, K): the smallest tile and one past its edges, K of one super-block, K
 # ends inside a group of K waves, then sizes wide enough for each larger tile
-# (32 x 128, 64 x 128, 64 x 256, 96 x 256, 128 x 256, 128 x 512).
+# (32 x 128, 64 x 128, 64 x 256, 96 x 256, 128 x 256, 128 x 512 or 256 x 256).
 # test_prefill_splits.py checks which tiles these reach.
 SHAPES = [(33, 64, 256), (64, 65, 512), (96, 63, 768), (65, 8201, 1280), (257, 4100, 512),
           (100, 22016, 512), (191, 22017, 768), (256, 22016, 256), (385, 22020, 512),
