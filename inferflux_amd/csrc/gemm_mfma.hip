@@ -524,10 +524,18 @@ static hipError_t launch_s(MfmaArgs &g, int count, bool f16, hipStream_t s) {
 //   Q4_K 22016 x 2048 at M = 60 (344)            27.3 / 26.3 / 30.4
 //   Q4_K 27648 x 5120 at M = 64 (432)            60.3 / 54.1 / 60.2
 //   Q8_0 2048 x 11008 at M = 60 (32)             93.5 / 81.4 / 74.9
+//   Q8_0 11008 x 2048 at M = 60 (172)            20.5 /      / 18.8
 //   Q8_0 22016 x 2048 at M = 64 (344)            27.6 / 29.6 / 33.7
+//   Q8_0 27648 x 5120 at M = 64 (432)            63.9 / 69.5
+//   Q8_0 20480 x 8192 at M = 60 (320)            88.7 / 100
 //   Q8_0 13824 x 5120 at M = 127 (432)           61.2 / 57.3 / 65.9
 // so Q8_0 (less unpacking to hide the loads behind) takes two groups only
-// from K = 4096 on.  Q6_K runs here on request only and keeps one group.
+// from K = 4096 on and where two tiles share their weights (M > 64).  Groups
+// need super-blocks enough: at K = 256 four took Q4_K 2048 x 256 from 5.0 to 6.5
+// and Q8_0 from 4.7 to 7.9, at K = 512 Q8_0 16384 x 512 from 8.1 to 9.5 (Q4_K 8.3, 8.5;
+// 2048 x 512 7.0, 6.9), at K = 1024 Q8_0 2048 x 1024 11.1 to 9.5; two at K = 768
+// Q4_K 24576 x 768 from 13.0 to 14.7.  Q6_K runs here on request only and keeps one
+// group.
 template <int QT>
 static hipError_t launch_qt(MfmaArgs &g, int count, bool f16, hipStream_t s) {
   int64_t big = 0, small = 0;
@@ -537,8 +545,9 @@ static hipError_t launch_qt(MfmaArgs &g, int count, bool f16, hipStream_t s) {
   }
   if (big >= 512 && g.M > 64) return launch_s<QT, 2, 1>(g, count, f16, s);
   if constexpr (QT != kTypeQ6_K) {
-    if (small <= 256) return launch_s<QT, 1, 4>(g, count, f16, s);
-    if (small <= 512 && (QT == kTypeQ4_K || g.K >= 4096))
+    constexpr bool q8 = QT == kTypeQ8_0;
+    if (small <= 256 && g.K >= (q8 ? 1024 : 512)) return launch_s<QT, 1, 4>(g, count, f16, s);
+    if (small > 256 && small <= 512 && g.K >= (q8 ? 4096 : 1024) && (!q8 || g.M > 64))
       return launch_s<QT, 1, 2>(g, count, f16, s);
   }
   return launch_s<QT, 1, 1>(g, count, f16, s);

@@ -24,14 +24,15 @@ def dev():
 # The bar is a part of a row's norm: Q4_K's fp16 activation sums alone are
 # 2^-11 of each min term off, which a row of a few outputs can fall short of,
 # so a Q4_K row has 63 outputs or more here (Q8_0 has no such term).
-# 64 x 64 tiles: up to 256 (four groups), 512 (two), more (one); 512 large
-# tiles with a batch of 64 and less stay on small ones
+# 64 x 64 tiles: up to 256 (four groups), 512 (two), more (one), and one with few
+# super-blocks; 512 large tiles with a batch of 64 and less stay on small ones
 CASES = [
     (Q4_K, 33, (63,), 256), (Q4_K, 64, (65, 63, 64), 768), (Q4_K, 65, (200, 130), 1280),
     (Q4_K, 95, (300,), 2048), (Q4_K, 40, (16389,), 512), (Q4_K, 64, (11000, 11009), 768),
     (Q4_K, 34, (32800,), 256), (Q4_K, 60, (65473,), 256), (Q4_K, 66, (65473,), 256),
     (Q8_0, 33, (1, 2, 3), 256), (Q8_0, 127, (513, 64), 1280), (Q8_0, 64, (65,), 768),
     (Q8_0, 63, (16500,), 4096), (Q8_0, 63, (16500,), 512), (Q8_0, 50, (65473,), 256),
+    (Q4_K, 64, (11000, 11009), 1280), (Q4_K, 40, (16389,), 1280), (Q8_0, 100, (8300,), 4352),
 ]
 
 

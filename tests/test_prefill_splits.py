@@ -95,6 +95,17 @@ def test_copy_ends_below_the_zero_offset(qt):
         assert ("k_q8_1_to_f16" in call) == bool(copied)
 
 
+@pytest.mark.parametrize("qt,M,N,K,groups", [
+    (Q4_K, 60, 2048, 256, 1), (Q4_K, 60, 2048, 512, 4), (Q4_K, 60, 16384, 768, 4),
+    (Q4_K, 60, 16385, 768, 1), (Q4_K, 60, 24576, 1024, 2), (Q4_K, 60, 32769, 2048, 1),
+    (Q8_0, 60, 2048, 256, 1), (Q8_0, 60, 16384, 768, 1), (Q8_0, 60, 16384, 1024, 4),
+    (Q8_0, 64, 27648, 5120, 1), (Q8_0, 65, 13824, 5120, 2), (Q8_0, 127, 16384, 3840, 1)])
+def test_int8_wave_groups(qt, M, N, K, groups):
+    """Few super-blocks, or weights that no second tile shares, keep one wave group."""
+    call = _instances("ifx_qgemm_prefill_kernel", qt, M, N, K, ops.PREFILL_INT8, 0)
+    assert call == [f"k_gemm_mfma<{qt},1,0>[{groups}]"]
+
+
 def test_int8_gpu_shapes_reach_every_group_count():
     from tests.test_gpu_mid_batch import CASES
     for qt in (Q4_K, Q8_0):
