@@ -67,10 +67,13 @@ namespace {
 // The tiles of launch_by_tile (rows, columns, K waves), and what a launch of
 // each costs by quant type (Q4_K, Q6_K, Q8_0): R rounds of 256 workgroups, one
 // a CU, and K values a workgroup take R (a + b K / 1024) + c w K / 1024 us, w
-// the rounds the workgroups fill.  Fitted to graph-replayed launches at M = 33
-// to 1999, N = 256 to 27648, K = 2048 to 27648 with HBM-cold weights (median
-// error 3 %).  One 256 x 256 tile for all of them, as before, took 65 us at
-// 173 x 11008 x 2048 (Q4_K; 26 now) and 147 at 512 x 5120 x 5120 (50): a grid of
+// the rounds the workgroups fill.  Fitted to launches with HBM-cold weights.  What
+// counts is the choice: over 3069 graph-replayed launches, all tiles at M = 33 to
+// 1999, N = 256 to 49152, K = 256 to 27648, the tile with the least cost took 1.007 of
+// the best one's time on average, 1.13 at most.  As times the figures are low, by 8 %
+// in the median (25 % for nine in ten: mostly K below 1024 and the small tiles).
+// One 256 x 256 tile with fp16 weights in LDS for all of them took 65 us at
+// 173 x 11008 x 2048 (Q4_K; 27 now) and 147 at 512 x 5120 x 5120 (50): a grid of
 // few workgroups leaves CUs idle, and a short batch pads the tile.
 struct TileInfo {
   int bm, bn, kw;
@@ -131,11 +134,13 @@ int max_splits(int count, const int *N, int M, int K) {
 
 // Tile and K splits of a launch: the cheapest by the table.  Only fp32 outputs
 // split (their partial sums meet in Y by atomics, or in slots), when the tiles
-// alone do not fill the CUs, up to max_splits; the reduction adds
-// about 4 us and 0.5 us a megabyte of partial sums.  A launch that would leave
-// three quarters of the CUs idle always splits.  splits_req > 0 forces the
-// count (tests; at most one split per group of stages).
-Plan f16_plan(int qt, bool f16, int count, const int *N, int M, int K, int splits_req) {
+// alone do not fill the CUs, up to max_splits; the reduction adds about 4 us and,
+// a megabyte of partial sums, 0.5 us with atomics and 0.25 in slots (planned alike,
+// the ordered 200 x 5120 x 5120 Q8_0 did not split, 44 us; in slots 37.)  What the
+// ordered plan does not split the other does not either, its splits cost more.
+// A launch that would leave three quarters of the CUs idle always splits.
+// splits_req > 0 forces the count (tests; at most one split per group of stages).
+Plan f16_plan(int qt, bool f16, bool ordered, int count, const int *N, int M, int K, int splits_req) {
   const int ty = qt == kTypeQ4_K ? 0 : qt == kTypeQ6_K ? 1 : 2;
   const int nch = K / kBK;
   const int forced = [] {  // IFX_F16_TILE (tuning)
@@ -172,7 +177,7 @@ Plan f16_plan(int qt, bool f16, int count, const int *N, int M, int K, int split
       const float k = static_cast<float>(std::min(p.spw * kc, nch) * kBK) / 1024.0f;
       float cost = rounds * (t.cost[ty].a + t.cost[ty].b * k) + t.cost[ty].c * w * k;
       if (in_order && t.kw > 1) cost *= kOrderedCost;
-      if (p.splits > 1) cost += 4.0f + 2e-6f * p.splits * static_cast<float>(n_sum) * M;
+      if (p.splits > 1) cost += 4.0f + (ordered ? 1e-6f : 2e-6f) * p.splits * static_cast<float>(n_sum) * M;
       if (best_cost == 0.0f || cost < best_cost) best_cost = cost, best = p;
     }
   }
@@ -184,7 +189,7 @@ Plan f16_plan(int qt, bool f16, int count, const int *N, int M, int K, int split
 hipError_t launch_qt(int qtype, int count, const void *const *W, const uint8_t *A, void *A16, void *const *Y,
                      const int *N, const void *bias, bool f16, int M, int K, int mode,
                      int splits_req, float *slots, hipStream_t s) {
-  const Plan p = f16_plan(qtype, f16, count, N, M, K, splits_req);
+  const Plan p = f16_plan(qtype, f16, slots != nullptr, count, N, M, K, splits_req);
   const TileInfo &t = kF16Tiles[p.tile];
   F16Args g{};
   for (int i = 0, end = 0; i < kMaxSeg; ++i) {
@@ -252,7 +257,7 @@ int64_t gemm_f16_workspace_bytes(int M, int K) {
 // Bytes of the ordered reduction's slots (splits x M x N fp32), or 0 when
 // the launch does not split K.
 int64_t gemm_f16_slot_bytes(int qtype, bool f16, int M, int N, int K) {
-  const int splits = f16_plan(qtype, f16, 1, &N, M, K, 0).splits;
+  const int splits = f16_plan(qtype, f16, true, 1, &N, M, K, 0).splits;
   return splits > 1 ? static_cast<int64_t>(splits) * M * N * 4 : 0;
 }
 

@@ -83,6 +83,25 @@ def test_other_launches_keep_the_k_waves(qt, M, N, K):
 
 
 @pytest.mark.parametrize("qt", [Q4_K, Q6_K, Q8_0])
+def test_ordered_launches_use_no_atomics(qt):
+    """The ordered entry splits into slots or not at all."""
+    Ms, Ns, Ks = [128, 200, 300, 512, 1024, 1999], [1, 300, 1024, 2048, 5120, 11008, 27648], [512, 2048, 5120, 11008]
+    split = 0
+    for M, N, K in itertools.product(Ms, Ns, Ks):
+        need = ops.prefill_ordered_workspace_bytes(qt, M, N, K)
+        call = _instances("ifx_qgemm_prefill_ordered", qt, M, N, K, "ws", need)
+        gemm = [k for k in call if k.startswith("k_gemm_f16<")]
+        epi = gemm[0].split("<")[1].split(",")[3]
+        assert len(gemm) == 1 and epi != "1" and "k_fill_zero" not in call, call
+        assert (epi == "2") == ("k_split_sum" in call), call
+        split += epi == "2"
+    assert split > 40
+    # wide enough for a split to gain in slots only
+    call = _instances("ifx_qgemm_prefill_ordered", Q8_0, 200, 5120, 5120, "ws", 1 << 40)
+    assert call[-1] == "k_split_sum"
+
+
+@pytest.mark.parametrize("qt", [Q4_K, Q6_K, Q8_0])
 def test_copy_ends_below_the_zero_offset(qt):
     """Chunks past K read zeros at byte 0xF0000000, so no fp16 copy reaches it."""
     N, K = 16384, 27648
