@@ -158,7 +158,8 @@ int ifx_qgemv(int quant_type, const void *W, const void *A_q8_1, void *Y, int ou
  * W_i [N[i]][K] and Y_i [M][N[i]].  For M <= 2 this is one launch whose
  * workgroups walk the rows of all projections, and so do the MFMA launches of
  * larger M.  mode: IFX_STORE or IFX_ACCUM (no bias).  W, Y and
- * N are host arrays of count entries.
+ * N are host arrays of count entries.  For M <= 32 the outputs must not
+ * overlap; above, projections whose outputs do run one after the other.
  * Replaces FusedQuantGemm::GemvQ8_1Pair / GemvQ8_1Triple
  * (fused_quant_gemm.h:272-276, 309-313; kernels mmvq.cuh:1197-1448). */
 int ifx_qgemv_grouped(int quant_type, int count, const void *const *W, void *const *Y,

@@ -398,6 +398,17 @@ int qgemv_impl(int quant_type, const void *W, const void *A_q8_1, void *Y, int o
   }
 }
 
+// Whether two of the projections write the same memory.  Their tiles may not
+// share a launch then: accumulated sums would race, and stores leave either.
+bool outputs_overlap(int count, void *const *Y, const int *N, bool f16, int M) {
+  const auto from = [&](int i) { return reinterpret_cast<uintptr_t>(Y[i]); };
+  const auto to = [&](int i) { return from(i) + uint64_t{f16 ? 2u : 4u} * M * N[i]; };
+  for (int i = 1; i < count; ++i)
+    for (int j = 0; j < i; ++j)
+      if (from(i) < to(j) && from(j) < to(i)) return true;
+  return false;
+}
+
 int grouped_impl(int quant_type, int count, const void *const *W, void *const *Y, const int *N,
                  const void *A_q8_1, int out_dtype, int mode, int M, int K, void *stream, void *ws,
                  int64_t ws_bytes, bool ordered) {
@@ -414,6 +425,14 @@ int grouped_impl(int quant_type, int count, const void *const *W, void *const *Y
   int n_total = 0;
   for (int i = 0; i < count; ++i) n_total += N[i];
   const Route r = route(quant_type, M, K, n_total, f16, true, !ordered && mode == IFX_ACCUM);
+  if ((r == Route::F16Gemm || r == Route::Mfma) && outputs_overlap(count, Y, N, f16, M)) {
+    for (int i = 0; i < count; ++i) {  // one after the other
+      const int rc = qgemv_impl(quant_type, W[i], A_q8_1, Y[i], out_dtype, mode, nullptr, M, N[i],
+                                K, stream, ws, ws_bytes, ordered);
+      if (rc != IFX_OK) return rc;
+    }
+    return IFX_OK;
+  }
   int wrc = IFX_OK;
   switch (r) {
   case Route::Gemv:

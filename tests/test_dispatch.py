@@ -124,3 +124,29 @@ def test_tiled_routing():
     assert rc == 0 and k == ["k_gemv_slot<8,8,1,0,0,0,1>"]
     rc, k = dry_dispatch("gemv", ops.Q8_0_T, 32, (151936,), 2048)  # >= 192 row groups: no split
     assert rc == 0 and k == ["k_gemv_dqr<8,0,1,0,4,2,8>"]
+
+
+@pytest.mark.parametrize("qt,M,K,f16", [(12, 60, 2048, False), (12, 512, 2048, False), (14, 64, 512, True),
+                                        (8, 64, 512, False), (8, 300, 1024, False)])
+@pytest.mark.parametrize("mode", ["STORE", "ACCUM"])
+def test_overlapping_outputs_run_in_order(qt, M, K, f16, mode):
+    """Above M = 32 projections that write the same memory do so one after the
+    other, in full or in part; outputs that only touch share a launch."""
+    from inferflux_amd import _lib, ops
+    L, N = _lib.load(), 256
+    size = M * N * (2 if f16 else 4)
+    W, NN = (_P * 3)(*[_fake(i) for i in range(3)]), (ctypes.c_int * 3)(N, N, N)
+    base = ctypes.cast(_fake(4), _P).value
+
+    def gemms(offs):
+        Y = (_P * 3)(*[base + o for o in offs])
+        with ops.launch_log(dry=True) as lg:
+            rc = L.ifx_qgemv_grouped(qt, 3, W, Y, NN, _fake(8), ops.OUT_F16 if f16 else ops.OUT_F32,
+                                     getattr(ops, mode), M, K, None)
+        assert rc == 0
+        return [k for k in lg.kernels if k.startswith("k_gemm_")]
+
+    assert len(gemms([0, size, 2 * size])) == 1
+    assert len(gemms([2 * size, 0, size])) == 1
+    for offs in ([0, 0, 0], [0, size, 0], [0, 2 * size, size + 2], [2 * size - 2, 0, size]):
+        assert len(gemms(offs)) == 3, offs
