@@ -32,9 +32,12 @@
 //      super-block, run on the matrix cores (v_mfma_f32_32x32x2f32) into
 //      the same accumulators, so it costs no VALU time.
 // This per-block rescaling (the activation d varies per row and per 32
-// values, the weight scale per column and per 32 values) is VALU work the
-// matrix cores cannot absorb: at three operations per output per block it
-// bounds the kernel near 15 % of the int8 MFMA peak.
+// values, the weight scale per column and per 32 values) is VALU work: at
+// three operations per output per block it bounds the kernel near 15 % of the
+// int8 MFMA peak.  Not the fewest possible at this exactness: fp16 operands sc q
+// (at most 945) and activation codes are whole numbers whose 32-value sums fp32
+// holds exactly, which leaves Q4_K one FMA per output and block at half the
+// matrix rate (not built).
 // MFMA lane layouts (32x32 output): lane l supplies row (l % 32) of A and
 // column (l % 32) of B for the K half (l / 32); it receives column l % 32
 // and rows 8*(i/4) + 4*(l/32) + (i%4), i = 0..15, of the result.
@@ -219,7 +222,13 @@ __global__ __launch_bounds__(256 * KW, KW == 1 ? 2 : 4) void k_gemm_mfma(MfmaArg
   constexpr int kBM = 64 * S, kBN = 64 * S;
   const int kg = KW == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x >> 8);
   Smem<QT, S> &sm = reinterpret_cast<Smem<QT, S> *>(smem_raw)[kg];
-  const int tid = threadIdx.x & 255;
+  // One group needs no mask, but the compiler allots registers and orders the loop
+  // by whether there is one.  us with / without: Q6_K 5120 x 27648 at M = 48
+  // 539 / 515, Q4_K 27648 x 5120 at M = 512 327 / 313, Q8_0 5120 x 5120 at
+  // M = 512 82.8 / 81.3; Q6_K on large tiles (fewer spills) 151936 x 2048 at
+  // M = 70 344 / 390, Q4_K on small ones 49152 x 512 at M = 60 14.6 / 14.8.
+  constexpr bool kMask = KW > 1 || (QT == kTypeQ6_K && S == 2) || (QT == kTypeQ4_K && S == 1);
+  const int tid = kMask ? threadIdx.x & 255 : threadIdx.x;
   const int lane = tid & 63;
   const int wave = tid >> 6;
   const int bx = blockIdx.x;
