@@ -249,14 +249,25 @@ __device__ __forceinline__ i32x4 w_operand(const WSb<QT> &w, int j) {
 // with KW = 4: 67 and 68 KB, two workgroups a CU) and gain all the same: us
 // without and with, 1024 x 5120 at M = 8 12.2 -> 9.2, 5120 x 5120 13.2 -> 12.1, fused
 // 11008 x 2048 19.4 -> 18.6, 2048 x 6144 26.3 -> 21.3.
-template <int KW, bool SW, bool TL>
-constexpr bool slot_staged() { return !TL && !(SW && KW == 8); }
+template <int KW, bool SW, bool TL, bool LN = false>
+constexpr bool slot_staged() { return !TL && !LN && !(SW && KW == 8); }
+
+// Whether a raw launch loads its weights in the lane layout after all (LN).  Going
+// through LDS delays a wave's first dot products, which Q4_K's short rows only
+// make up for where each wave walks a few super-blocks or eight waves share them
+// (Q6_K always does).  us lane layout / staged at M = 8: 2048 x 256 2.85 / 3.03,
+// 5120 x 512 3.51 / 3.68, 27648 x 1024 (accumulate) 7.1 / 7.6, at M = 4 the split
+// 2048 x 13824 9.3 / 9.6; but 2048 x 2048, eight waves of one super-block, 5 to 10 %
+// the other way.
+constexpr bool slot_lane_loads(int qtype, int kw, int ks, int nsb) {
+  return qtype == kTypeQ4_K && kw <= 4 && nsb <= kw * ks * (ks > 1 ? 2 : 1);
+}
 
 // NP: projections per workgroup (2 for the fused gate/up/SiLU launch).
-template <int QT, int MP, int KW, bool SW, bool TL>
+template <int QT, int MP, int KW, bool SW, bool TL, bool LN = false>
 constexpr int slot_lds_bytes() {
   constexpr int NP = SW ? 2 : 1;
-  constexpr int raw = slot_staged<KW, SW, TL>() ? NP * KW * WRaw<QT>::kArea : 0;  // first: 16-byte aligned
+  constexpr int raw = slot_staged<KW, SW, TL, LN>() ? NP * KW * WRaw<QT>::kArea : 0;  // first: 16-byte aligned
   constexpr int table = NP * KW * 2 * 8 * MP * 4;                     // per-wave d and s tables
   constexpr int red = NP * (KW > 1 ? KW - 1 : 0) * 64 * (MP / 2) * 4;  // partial results
   constexpr int gu = NP == 2 ? 2 * MP * 32 * 4 : 0;                    // gate/up outputs
@@ -279,13 +290,13 @@ constexpr int slot_lds_bytes() {
 // before the launch, or the bias) is loaded ahead of the weights, so the
 // epilogue waits on no dependent load (nothing else writes those outputs
 // during the launch: the same bits as 0).
-template <int QT, int MP, int KW, bool F16OUT, int SPLIT, bool SW = false, bool TL = false>
+template <int QT, int MP, int KW, bool F16OUT, int SPLIT, bool SW = false, bool TL = false, bool LN = false>
 __global__ __launch_bounds__(64 * KW * (SW ? 2 : 1)) void k_gemv_slot(const SlotArgs args) {
   using G = SlotGeo<QT, MP>;
   constexpr int NM = G::kNm;
   static_assert(!(SW && SPLIT), "the fused gate/up/SiLU launch does not split K");
   extern __shared__ __attribute__((aligned(16))) uint8_t smem_all[];
-  constexpr bool kStaged = slot_staged<KW, SW, TL>();
+  constexpr bool kStaged = slot_staged<KW, SW, TL, LN>();
   constexpr int kAreas = kStaged ? (SW ? 2 : 1) * KW * WRaw<QT>::kArea : 0;
   uint8_t *smem = smem_all + kAreas;  // past the waves' row areas
   const int bx = blockIdx.x;
@@ -688,6 +699,13 @@ template <int QT, int MP, int KW, bool F16OUT, int SPLIT, bool TL>
 void slot_launch(const SlotArgs &args, int blocks, int ks, hipStream_t s) {
   constexpr int lds = slot_lds_bytes<QT, MP, KW, false, TL>();
   slot_allow_lds<QT, MP, KW, F16OUT, SPLIT, false, TL>();
+  if constexpr (!TL && QT == kTypeQ4_K && KW <= 4) {
+    if (slot_lane_loads(QT, KW, ks, args.K >> 8)) {
+      IFX_LAUNCH(k_gemv_slot, (QT, MP, KW, F16OUT, SPLIT, false, false, true), dim3(blocks, ks),
+                 dim3(64 * KW), (slot_lds_bytes<QT, MP, KW, false, false, true>()), s, args);
+      return;
+    }
+  }
   if constexpr (TL)
     IFX_LAUNCH(k_gemv_slot, (QT, MP, KW, F16OUT, SPLIT, false, true), dim3(blocks, ks),
                dim3(64 * KW), lds, s, args);
