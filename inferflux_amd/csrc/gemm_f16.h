@@ -19,7 +19,7 @@
 // Why not int8: the per-32-value rescale of int8 MFMA results costs three
 // VALU operations per output per block and bounds that kernel near 15 % of
 // the int8 peak.  Dequantizing to fp16 costs about two VALU operations per
-// weight element per workgroup pass instead, independent of M.
+// weight element instead, once for all the batch rows of a tile (128 or 256 at most).
 //
 // How a workgroup works.  Its waves tile the output along n (each owns NT x 32
 // weight rows and all 32 MT batch rows of the tile) and, for small tiles, K:
@@ -443,8 +443,8 @@ __device__ __forceinline__ h8 w_slot(const LaneW<QT> &w, int sl) {
 // values the weights of that half and slot belong to.
 __device__ __forceinline__ int a_group(int sl, int h) { return 2 * sl + h; }
 
-// C consecutive outputs (m, n ..) = v by the launch's epilogue: 16-byte
-// accesses where the row pitch allows (g.vec), single ones at ragged edges.
+// C consecutive outputs (m, n ..) = v by the launch's epilogue, in 16-byte
+// accesses: of launches whose row pitch allows them (g.vec; C divides N).
 template <int C>
 __device__ __forceinline__ void put(const F16Args &g, void *Y, int N, int split, int m, int n,
                                     f32x4 (&v)[C / 4]) {
@@ -454,29 +454,18 @@ __device__ __forceinline__ void put(const F16Args &g, void *Y, int N, int split,
     if constexpr (C == 8) {
       uint16_t *p = static_cast<uint16_t *>(Y) + o;
       const uint16_t *bias = static_cast<const uint16_t *>(g.bias);
-      if (g.vec && n + C <= N) {
-        u32x4 t = {0, 0, 0, 0};
-        if (g.mode == 1) t = *reinterpret_cast<const u32x4 *>(p);
+      u32x4 t = {0, 0, 0, 0};
+      if (g.mode == 1) t = *reinterpret_cast<const u32x4 *>(p);
 #pragma unroll
-        for (int k = 0; k < 8; ++k) {
-          const uint32_t h = (t[k >> 1] >> (16 * (k & 1))) & 0xFFFFu;
-          if (g.mode == 1) v[k >> 2][k & 3] += h2f(h);
-          else if (g.mode == 2) v[k >> 2][k & 3] += h2f(bias[n + k]);
-        }
-#pragma unroll
-        for (int k = 0; k < 4; ++k)
-          t[k] = f2h_bits(v[k >> 1][2 * (k & 1)]) | f2h_bits(v[k >> 1][2 * (k & 1) + 1]) << 16;
-        *reinterpret_cast<u32x4 *>(p) = t;
-      } else {
-#pragma unroll
-        for (int k = 0; k < 8; ++k) {
-          if (n + k >= N) break;
-          float y = v[k >> 2][k & 3];
-          if (g.mode == 1) y += h2f(p[k]);
-          else if (g.mode == 2) y += h2f(bias[n + k]);
-          p[k] = static_cast<uint16_t>(f2h_bits(y));
-        }
+      for (int k = 0; k < 8; ++k) {
+        const uint32_t h = (t[k >> 1] >> (16 * (k & 1))) & 0xFFFFu;
+        if (g.mode == 1) v[k >> 2][k & 3] += h2f(h);
+        else if (g.mode == 2) v[k >> 2][k & 3] += h2f(bias[n + k]);
       }
+#pragma unroll
+      for (int k = 0; k < 4; ++k)
+        t[k] = f2h_bits(v[k >> 1][2 * (k & 1)]) | f2h_bits(v[k >> 1][2 * (k & 1) + 1]) << 16;
+      *reinterpret_cast<u32x4 *>(p) = t;
     }
     return;
   }
@@ -485,20 +474,9 @@ __device__ __forceinline__ void put(const F16Args &g, void *Y, int N, int split,
     float *p = static_cast<float *>(Y) + (slot ? static_cast<int64_t>(split) * g.M * N : 0) + o;
     const float *bias = static_cast<const float *>(g.bias);
     const int mode = slot ? 0 : g.mode;
-    if (g.vec && n + C <= N) {
-      if (mode == 1) v[0] += *reinterpret_cast<const f32x4 *>(p);
-      else if (mode == 2) v[0] += f32x4{bias[n], bias[n + 1], bias[n + 2], bias[n + 3]};
-      *reinterpret_cast<f32x4 *>(p) = v[0];
-    } else {
-#pragma unroll
-      for (int k = 0; k < 4; ++k) {
-        if (n + k >= N) break;
-        float y = v[0][k];
-        if (mode == 1) y += p[k];
-        else if (mode == 2) y += bias[n + k];
-        p[k] = y;
-      }
-    }
+    if (mode == 1) v[0] += *reinterpret_cast<const f32x4 *>(p);
+    else if (mode == 2) v[0] += f32x4{bias[n], bias[n + 1], bias[n + 2], bias[n + 3]};
+    *reinterpret_cast<f32x4 *>(p) = v[0];
   }
 }
 
@@ -738,25 +716,50 @@ __global__ __launch_bounds__(64 * WN * KW, 2) void k_gemm_f16(const F16Args g) {
       }
     }
   };
-  // atomic adds: a column a lane, so that a wave's adds fall on whole lines
-  auto add = [&](int i0) __attribute__((always_inline)) {
-    const float *bias = static_cast<const float *>(g.bias);
+  // Atomic adds, and stores to rows that do not start on 16 bytes: a column a
+  // lane, so that a wave's accesses fall on whole lines, and the sums of several
+  // rows read before the first is stored.  us with 4 or 8 single stores a lane / so:
+  // Q4_K 1905 x 30662 x 512 167 / 126 (a multiple of 8, 16-byte stores: 116),
+  // 743 x 16385 x 512 44 / 31, Q6_K 464 x 17874 x 1024 to fp16 59 / 47.
+  auto put_columns = [&](auto epi, int i0) __attribute__((always_inline)) {
+    constexpr int E = decltype(epi)::value, B = kRows / 2 < 8 ? kRows / 2 : 8;
+    using O = std::conditional_t<E == kEpiF16, uint16_t, float>;
+    const int row = m0 + 32 * i0 + kw * kRows + h, n = n_wave + l32;
+    O *y = static_cast<O *>(Y) + (E == kEpiSlot ? static_cast<int64_t>(split) * M * N : 0) +
+           static_cast<int64_t>(row) * N + n;
+    const bool with_y = (E == kEpiF32 || E == kEpiF16) && g.mode == 1;
+    const bool with_bias = E != kEpiSlot && g.mode == 2 && (E != kEpiAtomic || split == 0);
+    const auto f32 = [](O v) __attribute__((always_inline)) {
+      if constexpr (E == kEpiF16) return h2f(v);
+      else return v;
+    };
 #pragma unroll
-    for (int r0 = 0; r0 < kRows; r0 += 2) {
-      const int r = kw * kRows + r0 + h, rr = r & 31, m = m0 + 32 * i0 + r;
+    for (int r0 = 0; r0 < kRows; r0 += 2 * B) {
+      float v[B][NT];
 #pragma unroll
-      for (int j = 0; j < NT; ++j) {
-        const float *p = sum + wn * T::kPartF + ((r >> 5) * NT + j) * T::kTileF +
-                         64 * (4 * (rr >> 3) + (rr & 3)) + 32 * ((rr >> 2) & 1) + l32;
-        float v = p[0];
+      for (int b = 0; b < B; ++b)
 #pragma unroll
-        for (int c = 1; c < KW; ++c) v += p[c * WN * T::kPartF];
-        const int n = n_wave + 32 * j + l32;
-        if (m < M && n < N) {
-          if (g.mode == 2 && split == 0) v += bias[n];
-          atomicAdd(static_cast<float *>(Y) + static_cast<int64_t>(m) * N + n, v);
+        for (int j = 0; j < NT; ++j) {
+          const int r = kw * kRows + r0 + 2 * b + h, rr = r & 31;
+          const float *p = sum + wn * T::kPartF + ((r >> 5) * NT + j) * T::kTileF +
+                           64 * (4 * (rr >> 3) + (rr & 3)) + 32 * ((rr >> 2) & 1) + l32;
+          v[b][j] = p[0];
+#pragma unroll
+          for (int c = 1; c < KW; ++c) v[b][j] += p[c * WN * T::kPartF];
         }
-      }
+#pragma unroll
+      for (int b = 0; b < B; ++b)
+#pragma unroll
+        for (int j = 0; j < NT; ++j)
+          if (row + r0 + 2 * b < M && n + 32 * j < N) {
+            O *o = y + static_cast<int64_t>(r0 + 2 * b) * N + 32 * j;
+            float t = v[b][j];
+            if (with_y) t += f32(*o);
+            if (with_bias) t += f32(static_cast<const O *>(g.bias)[n + 32 * j]);
+            if constexpr (E == kEpiAtomic) atomicAdd(o, t);
+            else if constexpr (E == kEpiF16) *o = static_cast<uint16_t>(f2h_bits(t));
+            else *o = t;
+          }
     }
   };
   auto pass = [&](auto first) __attribute__((always_inline)) {
@@ -775,7 +778,10 @@ __global__ __launch_bounds__(64 * WN * KW, 2) void k_gemm_f16(const F16Args g) {
           for (int e = 0; e < 16; ++e) d[(i * NT + j) * T::kTileF + 64 * e] = acc[i0 + i][j][e];
       if constexpr (KW > 1) __syncthreads();
       else wave_sync();
-      if (g.epi == kEpiAtomic) add(i0);
+      if (g.epi == kEpiAtomic) put_columns(std::integral_constant<int, kEpiAtomic>{}, i0);
+      else if (!g.vec && g.epi == kEpiF16) put_columns(std::integral_constant<int, kEpiF16>{}, i0);
+      else if (!g.vec && g.epi == kEpiSlot) put_columns(std::integral_constant<int, kEpiSlot>{}, i0);
+      else if (!g.vec) put_columns(std::integral_constant<int, kEpiF32>{}, i0);
       else if (g.epi == kEpiF16) store(std::integral_constant<int, 8>{}, i0);
       else store(std::integral_constant<int, 4>{}, i0);
     }

@@ -149,3 +149,32 @@ def test_prefill_wide_splits(orc, dev, qtype, M, N, K):
         ops.qgemm_prefill_ordered(qtype, W, A, M, N, K, ws, out=y, mode=ops.ACCUM)
     assert ",2,0>" in lg.kernels[0] and lg.kernels[1] == "k_split_sum", lg.kernels
     check_rows(down(y)[:, idx], ye + 1.0)
+
+
+# Rows that do not start on 16 bytes, on tiles with one, two, four and eight K waves
+@pytest.mark.parametrize("qtype,M,N,K", [
+    (Q4_K, 130, 16385, 256), (Q4_K, 743, 16385, 512), (Q6_K, 600, 12290, 512), (Q6_K, 300, 6146, 512), (Q6_K, 65, 4101, 256),
+    (Q8_0, 600, 12290, 512), (Q8_0, 257, 8201, 320), (Q8_0, 129, 1027, 192), (Q4_K, 97, 70, 256),
+])
+@pytest.mark.parametrize("f16", [False, True])
+def test_prefill_unaligned_rows(orc, dev, qtype, M, N, K, f16):
+    """Stored, added to what is there, and with a bias: the same sums each time."""
+    import torch
+    from inferflux_amd import ops, synth
+    note(f"prefill unaligned rows type={qtype} M={M} N={N} K={K} f16={f16}")
+    w = synth.blocks(qtype, N, K, seed=N + K)
+    a = orc.quantize_q8_1(synth.activations(M, K, seed=M + K, outlier_frac=0.01))
+    W, A, f = up(w, dev), up(a, dev), ops.PREFILL_F16
+    dt = torch.float16 if f16 else torch.float32
+    y = ops.qgemm_prefill_kernel(qtype, W, A, M, N, K, f, splits=1)
+    idx = np.unique(np.concatenate([[0, 31, 32, N - 1], np.random.default_rng(N).choice(N, min(N, 96))]))
+    check_rows(down(y)[:, idx], orc.gemv_exact(qtype, w[idx], a, M, len(idx), K))
+    rng = torch.Generator().manual_seed(N)
+    base = torch.randn(M, N, generator=rng).to(dt).to(dev)
+    bias = torch.randn(N, generator=rng).to(dt).to(dev)
+    got = ops.qgemm_prefill_kernel(qtype, W, A, M, N, K, f, splits=1, out_dtype=dt)
+    assert torch.equal(got, y.to(dt))  # one rounding of the same fp32 sum
+    got = ops.qgemm_prefill_kernel(qtype, W, A, M, N, K, f, splits=1, out=base.clone(), mode=ops.ACCUM)
+    assert torch.equal(got, (y + base.float()).to(dt))
+    got = ops.qgemm_prefill_kernel(qtype, W, A, M, N, K, f, splits=1, out_dtype=dt, mode=ops.BIAS, bias=bias)
+    assert torch.equal(got, (y + bias.float()).to(dt))
