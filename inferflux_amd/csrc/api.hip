@@ -143,13 +143,13 @@ namespace {
 constexpr int kMaxGemvMDefault = 2;
 constexpr int kMaxSkinnyM = 32;
 // Prefill kernel for M > 32: the fp16 GEMM from min_f16_gemm_m(qtype) rows
-// on, else the int8 MFMA GEMM.  Measured at the 32B shapes (graph-replayed,
-// us for fp16 / int8): Q6_K 5120 x 27648 M = 48: 111 / 438, M = 128: 118 /
-// 438 (the int8 kernel's per-block rescale of 16-value Q6_K groups); Q4_K
-// 27648 x 5120 M = 48: 104 / 63, M = 64: 98 / 64, M = 96: 99 / 105, M = 128:
-// 102 / 104 (fp16 on a 256 x 256 tile).  Batches under the lines keep the
-// integer-exact sums whatever the fp16 kernel's time.  IFX_PREFILL=int8|f16
-// forces one (tuning; read once).
+// on, else the int8 MFMA GEMM.  us for fp16 / int8 (graph-replayed, both on the
+// present tiles): Q6_K 5120 x 27648 M = 48 57 / 515, M = 128 83 / 514; Q4_K
+// 27648 x 5120 M = 48 44 / 55, M = 64 42 / 55, M = 96 57 / 101, M = 128 59 / 103;
+// Q8_0 27648 x 5120 M = 64 56 / 62, M = 127 87 / 105; 11008 x 2048 Q4_K M = 60
+// 16 / 17, Q8_0 M = 96 25 / 26.  The lines are older than the fp16 tiles for short
+// batches: under them the integer-exact sums are kept, faster or not.
+// IFX_PREFILL=int8|f16 forces one (tuning; read once).
 int min_f16_gemm_m(int qtype) {
   return qtype == IFX_TYPE_Q6_K ? kMaxSkinnyM + 1 : qtype == IFX_TYPE_Q4_K ? 96 : 128;
 }
@@ -812,8 +812,8 @@ int ifx_qgemm_prefill(int quant_type, const void *W, const void *A_q8_1, void *Y
 
 // The fp16 copy is used where many weight tiles share it.  The line is part
 // of the interface (callers size their workspace by it); on the present tiles
-// the GEMM gains little by it (Q4_K 27648 x 5120 at M = 512: 163-171 us
-// without, 162 with), on few tiles the copy's own launch costs more.
+// the GEMM gains little by it (Q4_K 27648 x 5120 at M = 512: 162 us
+// without, 155 with), on few tiles the copy's own launch costs more.
 constexpr int kMinWorkspaceN = 16384;
 
 int64_t ifx_qgemm_prefill_workspace_bytes(int quant_type, int M, int N, int K) {

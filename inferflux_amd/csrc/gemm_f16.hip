@@ -32,7 +32,7 @@ __global__ __launch_bounds__(256) void k_q8_1_to_f16(const uint8_t *__restrict__
   out[t] = u32x4{o[0], o[1], o[2], o[3]};
 }
 
-// The ordered reduction of the SPL = 2 GEMM: y = ((s_0 + s_1) + ...) over
+// The ordered reduction of a launch with slots: y = ((s_0 + s_1) + ...) over
 // the splits' slots in split order, then the epilogue (mode 1: + Y, 2:
 // + bias[n]).  Four consecutive outputs per thread (16-byte accesses when
 // M * N % 4 == 0 and Y is 16-byte aligned).
