@@ -258,7 +258,8 @@ constexpr bool slot_staged() { return !TL && !LN && !(SW && KW == 8); }
 // (Q6_K always does).  us lane layout / staged at M = 8: 2048 x 256 2.85 / 3.03,
 // 5120 x 512 3.51 / 3.68, 27648 x 1024 (accumulate) 7.1 / 7.6, at M = 4 the split
 // 2048 x 13824 9.3 / 9.6; but 2048 x 2048, eight waves of one super-block, 5 to 10 %
-// the other way.
+// the other way.  The fused launch does so where it has one or two waves a
+// projection: 6144 x 256 3.40 / 3.58, 6144 x 768 at M = 4 5.32 / 5.55.
 constexpr bool slot_lane_loads(int qtype, int kw, int ks, int nsb) {
   return qtype == kTypeQ4_K && kw <= 4 && nsb <= kw * ks * (ks > 1 ? 2 : 1);
 }
@@ -778,6 +779,10 @@ void slot_swiglu_launch(const SlotArgs &args, bool f16h, hipStream_t s) {
   if constexpr (TL) {
     if (f16h) IFX_LAUNCH(k_gemv_slot, (QT, MP, KW, true, false, true, true), grid, dim3(128 * KW), lds, s, args);
     else IFX_LAUNCH(k_gemv_slot, (QT, MP, KW, false, false, true, true), grid, dim3(128 * KW), lds, s, args);
+  } else if constexpr (QT == kTypeQ4_K && KW <= 2) {  // up to three super-blocks a row (slot_lane_loads)
+    constexpr int ln = slot_lds_bytes<QT, MP, KW, true, false, true>();
+    if (f16h) IFX_LAUNCH(k_gemv_slot, (QT, MP, KW, true, false, true, false, true), grid, dim3(128 * KW), ln, s, args);
+    else IFX_LAUNCH(k_gemv_slot, (QT, MP, KW, false, false, true, false, true), grid, dim3(128 * KW), ln, s, args);
   } else {
     if (f16h) IFX_LAUNCH(k_gemv_slot, (QT, MP, KW, true, false, true), grid, dim3(128 * KW), lds, s, args);
     else IFX_LAUNCH(k_gemv_slot, (QT, MP, KW, false, false, true), grid, dim3(128 * KW), lds, s, args);
